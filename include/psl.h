@@ -261,11 +261,14 @@ int psl_grid_check_health(psl_grid* grid, int64_t* bad_cells, double* rho_min, d
 /* Many independent grids advanced together (no reference counterpart: the
  * reference steps one grid at a time).  Each grid keeps its own flags, given
  * values, Cs (uniform or per cell) and storage (all grids share the storage);
- * one step of all grids is a device shift update, one bulk launch over the
- * blocks of every grid and one launch over all boundary lists (or one fused
- * launch).  Steps are captured in hipGraphs of one step and of
- * steps_per_graph steps (default 1000) and replayed, so nsteps steps take
- * nsteps / steps_per_graph + nsteps % steps_per_graph graph launches.  Every
+ * one step of all grids is one bulk launch over the blocks of every grid and
+ * one launch over all boundary lists (or one fused launch).  Steps are captured
+ * in hipGraphs of one step and of steps_per_graph steps (default 1000) and
+ * replayed, so nsteps steps take nsteps / steps_per_graph + nsteps %
+ * steps_per_graph graph launches; a batch whose distributions exceed 192 MB
+ * instead takes calls of several steps in groups of grids that fit the
+ * last-level cache, all steps of one group after the other, launched without
+ * a graph.  Every
  * grid's result is bit-identical to stepping it alone.  Grids need flags and
  * must not use periodic copies, sub-grids or a learned closure (checked at
  * every psl_batch_step).  The grids' own handles stay valid (get_f,

@@ -18,10 +18,15 @@
 //
 // The per-cell work is bulk_update / boundary_update, the same functions on
 // the same StepParams / BoundaryParams as the single-grid kernels, so every
-// grid's result is bit-identical to stepping it alone.  Steps are captured
-// in hipGraphs, one of a single step and one of steps_per_graph (default
-// 1000) consecutive steps, and replayed: 5000 steps are five graph launches
-// whatever the number of grids.  The block order of the grids (as given, or largest
+// grid's result is bit-identical to stepping it alone.
+//
+// What bounds a step is the traffic of the distributions, so a batch larger
+// than the last-level cache runs in groups of grids that fit it together: each
+// group takes all the steps of the call before the next one starts (grids are
+// independent), and its populations then come from the cache in every step but
+// the first.  A batch that fits, or a call of one step, runs all grids in each
+// launch, from hipGraphs: one of a single step and one of steps_per_graph
+// (default 1000) consecutive steps.  The block order of the grids (as given, or largest
 // first) and the kernel variant are chosen by psl_batch_autotune, and with
 // them the cells per thread and the tile order by psl_batch_autotune_layouts.
 #include "psl_internal.h"
@@ -33,27 +38,60 @@
 
 namespace psl {
 
-// applyStreaming of every grid (include/applyStreaming.h:11-31) and the
-// per-population stream bases of the step.
+// Streaming of grid d (include/applyStreaming.h:11-31): moves the shift of
+// population q on and writes the step's stream bases into P.
 template <class St>
-__global__ void k_batch_advance(StepParams* __restrict__ params, const void* const* __restrict__ fbase,
-                                const int* __restrict__ delta, int* __restrict__ shift, int nd) {
+__device__ __forceinline__ void advance_one(StepParams& P, const void* fbase, const int* delta, int* shift, int q) {
   typedef typename St::T T;
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nd * 27) return;
-  const int d = t / 27, q = t - d * 27;
-  StepParams& P = params[d];
   const int64_t N = P.n;
-  int64_t s = shift[t];
-  s -= delta[t];
+  int64_t s = shift[q];
+  s -= delta[q];
   // reduced modulo N (also on grids thinner than two wraps allow)
   s %= N;
   if (s < 0) s += N;
-  shift[t] = (int)s;
-  T* row = (T*)fbase[d] + (size_t)q * P.n + s;
+  shift[q] = (int)s;
+  T* row = (T*)fbase + (size_t)q * P.n + s;
   P.lo[q] = row;
   P.hi[q] = row - P.n;
   P.thr[q] = P.n - (uint32_t)s;
+}
+
+// Streaming of the grids dom[0 .. nd) ahead of the first step of a run.
+template <class St>
+__global__ void k_batch_advance(StepParams* __restrict__ params, const void* const* __restrict__ fbase,
+                                const int* __restrict__ delta, int* __restrict__ shift,
+                                const uint32_t* __restrict__ dom, int nd) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= nd * 27) return;
+  const int g = t / 27, q = t - g * 27;
+  const uint32_t d = dom[g];
+  advance_one<St>(params[d], fbase[d], delta + 27 * d, shift + 27 * d, q);
+}
+
+// Streaming of the step after this one, by one workgroup past the step's own
+// (block nb of the launch): the steps of a run take the two parameter tables
+// in turn, so nothing in flight reads what it writes, and a step is spared a
+// launch of its own for 27 shifts per grid (5 us; it matters where a step of
+// one group of grids takes 60).  A workgroup of its own, because a store to a
+// parameter table ahead of the update in the same workgroup keeps the
+// compiler from reading the tables through the scalar cache (the 60-domain
+// step then took 2.64 ms instead of 1.40).  The run's last
+// step is launched without it.
+struct NextStep {
+  StepParams* next;
+  const void* const* fbase;
+  const int* delta;
+  int* shift;
+  const uint32_t* dom;
+  uint32_t nd;
+  uint32_t nb;  // workgroups of the step itself
+};
+template <class St>
+__device__ __forceinline__ void advance_next(const NextStep& nx) {
+  for (uint32_t t = threadIdx.x; t < nx.nd * 27u; t += 256u) {
+    const uint32_t g = t / 27u, q = t - g * 27u, d = nx.dom[g];
+    advance_one<St>(nx.next[d], nx.fbase[d], nx.delta + 27 * d, nx.shift + 27 * d, (int)q);
+  }
 }
 
 // One tile of CPT consecutive 256-cell blocks of grid tile_domain[t], its
@@ -62,8 +100,13 @@ __global__ void k_batch_advance(StepParams* __restrict__ params, const void* con
 template <class St, int TUNE, int CPT>
 __global__ __launch_bounds__(256) void k_batch_bulk(const StepParams* __restrict__ params,
                                                     const uint32_t* __restrict__ tile_domain,
-                                                    const uint32_t* __restrict__ tile_index, uint32_t remap) {
-  const uint32_t t = remap ? xcd_block_chunked<64>(blockIdx.x, gridDim.x) : blockIdx.x;
+                                                    const uint32_t* __restrict__ tile_index, uint32_t remap,
+                                                    NextStep nx) {
+  if (blockIdx.x == nx.nb) {
+    advance_next<St>(nx);
+    return;
+  }
+  const uint32_t t = remap ? xcd_block_chunked<64>(blockIdx.x, nx.nb) : blockIdx.x;
   const uint32_t d = tile_domain[t];
   const uint32_t first = tile_index[t] * CPT;
   for (int k = 0; k < CPT; ++k) bulk_update<St, true, true, TUNE>(params[d], first + k);
@@ -73,9 +116,10 @@ template <class St>
 __global__ __launch_bounds__(256) void k_batch_boundary(const StepParams* __restrict__ params,
                                                         const BoundaryParams* __restrict__ bparams,
                                                         const uint32_t* __restrict__ bblock_domain,
-                                                        const uint32_t* __restrict__ bblock_first) {
-  const uint32_t d = bblock_domain[blockIdx.x];
-  boundary_update<St>(params[d], bparams[d], (blockIdx.x - bblock_first[d]) * 256u + threadIdx.x);
+                                                        const uint32_t* __restrict__ bblock_first, uint32_t b0) {
+  const uint32_t b = b0 + blockIdx.x;
+  const uint32_t d = bblock_domain[b];
+  boundary_update<St>(params[d], bparams[d], (b - bblock_first[d]) * 256u + threadIdx.x);
 }
 
 // One workgroup of the fused batch launch: entry `e` of grid `d`'s fused
@@ -91,8 +135,12 @@ struct BatchEntry {
 template <class St, int TUNE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_batch_fused(
     const StepParams* __restrict__ params, const BoundaryParams* __restrict__ bparams,
-    const BatchEntry* __restrict__ order, uint32_t remap) {
-  const uint32_t w = remap ? xcd_block_chunked<64>(blockIdx.x, gridDim.x) : blockIdx.x;
+    const BatchEntry* __restrict__ order, uint32_t remap, NextStep nx) {
+  if (blockIdx.x == nx.nb) {
+    advance_next<St>(nx);
+    return;
+  }
+  const uint32_t w = remap ? xcd_block_chunked<64>(blockIdx.x, nx.nb) : blockIdx.x;
   const BatchEntry x = order[w];
   if (x.e.b != FUSED_BULK) {
     BoundaryParams b = bparams[x.d];
@@ -107,6 +155,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k
 
 using namespace psl;
 
+namespace {
+// Distributions stepped together at most, so that they stay in the 256 MB
+// last-level cache from one step to the next.  60 channels of 2.4 GB in FP16,
+// 100 steps: 1.40 ms per step with every grid in each launch; in groups of at
+// most 128 / 160 / 192 / 224 MB 1.26 / 1.17 / 1.09 / 1.08 ms (two launches)
+// and 1.19 / 1.11 / 1.06 / 1.17 ms (fused).  Smaller groups pay more launches,
+// at 224 MB the tables, flags and the drag samples' reads start to evict.
+constexpr size_t GROUP_BYTES = (size_t)192 << 20;
+// Consecutive grids of the launch order that are stepped together: their
+// ranges of the launch tables.
+struct BatchGroup {
+  uint32_t dom0 = 0, ndom = 0;      // launch order
+  uint32_t tile0 = 0, ntile = 0;    // bulk tiles
+  uint32_t bblk0 = 0, nbblk = 0;    // boundary blocks
+  uint32_t fused0 = 0, nfused = 0;  // fused order
+};
+}  // namespace
+
 struct psl_batch {
   std::vector<psl_grid*> grids;
   int storage = PSL_F32;
@@ -115,11 +181,12 @@ struct psl_batch {
   int cpt = 1;         // cells per thread of the two-launch bulk kernel (1 or 2)
   int tile_order = 0;  // 0: each grid's tiles in turn, 1: interleaved across grids
   hipStream_t stream = nullptr;
-  StepParams* d_params = nullptr;
+  StepParams* d_params = nullptr;  // two tables of one entry per grid, used in turn
   BoundaryParams* d_bparams = nullptr;
   const void** d_fbase = nullptr;
   int* d_delta = nullptr;
   int* d_shift = nullptr;
+  uint32_t* d_dom = nullptr;           // launch order -> grid
   uint32_t* d_block_domain = nullptr;  // bulk tile -> grid
   uint32_t* d_block_tile = nullptr;    // bulk tile -> tile index within its grid
   uint32_t* d_bblock_domain = nullptr;
@@ -127,6 +194,8 @@ struct psl_batch {
   BatchEntry* d_order = nullptr;
   uint32_t total_blocks = 0, total_bblocks = 0, total_bnd = 0, total_fused = 0;
   int64_t total_cells = 0;
+  BatchGroup whole;                // all grids
+  std::vector<BatchGroup> groups;  // at least one
   hipGraph_t graph = nullptr;  // one step
   hipGraphExec_t exec = nullptr;
   int steps_per_graph = 1000;  // steps captured in graph_k
@@ -154,7 +223,8 @@ void free_graphs(psl_batch* b) {
 void free_batch_device(psl_batch* b) {
   free_graphs(b);
   void* ptrs[] = {b->d_params,       b->d_bparams,     b->d_fbase,         b->d_delta,          b->d_shift,
-                  b->d_block_domain, b->d_block_tile, b->d_bblock_domain, b->d_bblock_first, b->d_order};
+                  b->d_block_domain, b->d_block_tile, b->d_bblock_domain, b->d_bblock_first, b->d_order,
+                  b->d_dom};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   b->d_params = nullptr;
@@ -167,18 +237,26 @@ void free_batch_device(psl_batch* b) {
   b->d_bblock_domain = nullptr;
   b->d_bblock_first = nullptr;
   b->d_order = nullptr;
+  b->d_dom = nullptr;
 }
 
+// Step s of a run of `steps` steps of one group of grids.
 template <class St>
-int enqueue_step(psl_batch* b) {
-  const int nd = (int)b->grids.size();
-  k_batch_advance<St><<<(nd * 27 + 255) / 256, 256, 0, b->stream>>>(b->d_params, b->d_fbase, b->d_delta,
-                                                                     b->d_shift, nd);
+int enqueue_step(psl_batch* b, const BatchGroup& G, int s, int steps) {
+  const size_t nd = b->grids.size();
+  const StepParams* params = b->d_params + (s & 1) * nd;
+  if (s == 0)
+    k_batch_advance<St><<<(G.ndom * 27 + 255) / 256, 256, 0, b->stream>>>(
+        b->d_params, b->d_fbase, b->d_delta, b->d_shift, b->d_dom + G.dom0, (int)G.ndom);
+  const bool fused = (b->tuning & PSL_TUNE_FUSED_BOUNDARY) && b->total_bnd;
+  const uint32_t nb = fused ? G.nfused : G.ntile;
+  const uint32_t launch = s + 1 < steps ? nb + 1 : nb;
+  const NextStep nx{b->d_params + ((s + 1) & 1) * nd, b->d_fbase, b->d_delta, b->d_shift, b->d_dom + G.dom0, G.ndom, nb};
   const uint32_t remap = (b->tuning & PSL_TUNE_XCD_REMAP) ? 1u : 0u;
   const int nt = b->tuning & (TUNE_NT_LOAD | TUNE_NT_STORE);
-  if ((b->tuning & PSL_TUNE_FUSED_BOUNDARY) && b->total_bnd) {
+  if (fused) {
 #define PSL_FUSED(V) \
-  k_batch_fused<St, V><<<b->total_fused, 256, 0, b->stream>>>(b->d_params, b->d_bparams, b->d_order, remap)
+  k_batch_fused<St, V><<<launch, 256, 0, b->stream>>>(params, b->d_bparams, b->d_order + G.fused0, remap, nx)
     switch (nt) {
       case 0: PSL_FUSED(0); break;
       case 1: PSL_FUSED(1); break;
@@ -187,9 +265,9 @@ int enqueue_step(psl_batch* b) {
     }
 #undef PSL_FUSED
   } else {
-#define PSL_BULK(V, C)                                                                                          \
-  k_batch_bulk<St, V, C><<<b->total_blocks, 256, 0, b->stream>>>(b->d_params, b->d_block_domain, b->d_block_tile, \
-                                                                 remap)
+#define PSL_BULK(V, C)                                                                                     \
+  k_batch_bulk<St, V, C><<<launch, 256, 0, b->stream>>>(params, b->d_block_domain + G.tile0, b->d_block_tile + G.tile0, \
+                                                         remap, nx)
     if (b->cpt == 2) {
       switch (nt) {
         case 0: PSL_BULK(0, 2); break;
@@ -206,20 +284,22 @@ int enqueue_step(psl_batch* b) {
       }
     }
 #undef PSL_BULK
-    if (b->total_bnd)
-      k_batch_boundary<St><<<b->total_bblocks, 256, 0, b->stream>>>(b->d_params, b->d_bparams, b->d_bblock_domain,
-                                                                     b->d_bblock_first);
+    if (G.nbblk)
+      k_batch_boundary<St><<<G.nbblk, 256, 0, b->stream>>>(params, b->d_bparams, b->d_bblock_domain,
+                                                           b->d_bblock_first, G.bblk0);
   }
   PSL_LAUNCH_CHECK();
   return PSL_OK;
 }
 
-int enqueue_dispatch(psl_batch* b) {
-  switch (b->storage) {
-    case PSL_F32: return enqueue_step<StF32>(b);
-    case PSL_F16DEV: return enqueue_step<StF16>(b);
-    default: return enqueue_step<StBF16>(b);
-  }
+int enqueue_run(psl_batch* b, const BatchGroup& G, int steps) {
+  int rc = PSL_OK;
+  for (int s = 0; s < steps && rc == PSL_OK; ++s) switch (b->storage) {
+      case PSL_F32: rc = enqueue_step<StF32>(b, G, s, steps); break;
+      case PSL_F16DEV: rc = enqueue_step<StF16>(b, G, s, steps); break;
+      default: rc = enqueue_step<StBF16>(b, G, s, steps); break;
+    }
+  return rc;
 }
 
 template <class T>
@@ -239,7 +319,7 @@ int capture_steps(psl_batch* b, int steps, hipGraph_t* graph_out, hipGraphExec_t
   b->stream = cap;
   hipError_t e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
   int rc = PSL_OK;
-  for (int s = 0; e == hipSuccess && rc == PSL_OK && s < steps; ++s) rc = enqueue_dispatch(b);
+  if (e == hipSuccess) rc = enqueue_run(b, b->whole, steps);
   hipGraph_t graph = nullptr;
   hipError_t e2 = hipStreamEndCapture(cap, &graph);
   b->stream = saved;
@@ -311,36 +391,69 @@ int build_batch(psl_batch* b) {
     ntile[d] = (uint32_t)((b->grids[d]->info.cellCount + tile_cells - 1) / tile_cells);
     max_tiles = std::max(max_tiles, ntile[d]);
   }
-  if (b->tile_order == 1) {
-    for (uint32_t t = 0; t < max_tiles; ++t)
-      for (int d : order)
-        if (t < ntile[d]) {
-          block_domain.push_back((uint32_t)d);
+  // groups of consecutive grids of the launch order whose distributions fit
+  // GROUP_BYTES together (a larger grid is a group of its own), of about equal size
+  std::vector<uint32_t> dom(order.begin(), order.end());
+  const size_t cell_bytes = 27 * storage_bytes(b->storage);
+  auto bytes_of = [&](int d) { return (size_t)b->grids[d]->info.cellCount * cell_bytes; };
+  size_t total_bytes = 0;
+  for (int d : order) total_bytes += bytes_of(d);
+  const size_t want = (total_bytes + GROUP_BYTES - 1) / GROUP_BYTES;
+  const size_t share = (total_bytes + want - 1) / want;
+  std::vector<size_t> ends;  // launch-order positions past each group
+  size_t in_group = 0, before = 0;
+  for (int at = 0; at < nd; ++at) {
+    const size_t bytes = bytes_of(order[at]);
+    if (in_group && (in_group + bytes > GROUP_BYTES || before + bytes / 2 > share * (ends.size() + 1))) {
+      ends.push_back((size_t)at);
+      in_group = 0;
+    }
+    in_group += bytes;
+    before += bytes;
+  }
+  ends.push_back((size_t)nd);
+  std::vector<BatchEntry> fused;
+  size_t at0 = 0;
+  b->groups.clear();
+  for (size_t end : ends) {
+    BatchGroup G;
+    G.dom0 = (uint32_t)at0;
+    G.ndom = (uint32_t)(end - at0);
+    G.tile0 = (uint32_t)block_domain.size();
+    if (b->tile_order == 1) {
+      for (uint32_t t = 0; t < max_tiles; ++t)
+        for (size_t at = at0; at < end; ++at)
+          if (t < ntile[order[at]]) {
+            block_domain.push_back((uint32_t)order[at]);
+            block_tile.push_back(t);
+          }
+    } else {
+      for (size_t at = at0; at < end; ++at)
+        for (uint32_t t = 0; t < ntile[order[at]]; ++t) {
+          block_domain.push_back((uint32_t)order[at]);
           block_tile.push_back(t);
         }
-  } else {
-    for (int d : order)
-      for (uint32_t t = 0; t < ntile[d]; ++t) {
-        block_domain.push_back((uint32_t)d);
-        block_tile.push_back(t);
-      }
-  }
-  for (int d : order) {
-    const psl_grid* g = b->grids[d];
-    const uint32_t nbb = (g->n_bc + 255u) / 256u;
-    bblock_first[d] = (uint32_t)bblock_domain.size();
-    bblock_domain.insert(bblock_domain.end(), nbb, (uint32_t)d);
-  }
-  // the fused order: every grid's own interleaving, grids in launch order
-  std::vector<BatchEntry> fused;
-  for (int d : order) {
-    const psl_grid* g = b->grids[d];
-    if (g->fused_host.empty()) {
-      const uint32_t nbk = (uint32_t)((g->info.cellCount + 255) / 256);
-      for (uint32_t k = 0; k < nbk; ++k) fused.push_back({(uint32_t)d, {k, FUSED_BULK}, 0u});
-    } else {
-      for (const FusedEntry& e : g->fused_host) fused.push_back({(uint32_t)d, e, 0u});
     }
+    G.ntile = (uint32_t)block_domain.size() - G.tile0;
+    G.bblk0 = (uint32_t)bblock_domain.size();
+    G.fused0 = (uint32_t)fused.size();
+    for (size_t at = at0; at < end; ++at) {
+      const int d = order[at];
+      const psl_grid* g = b->grids[d];
+      bblock_first[d] = (uint32_t)bblock_domain.size();
+      bblock_domain.insert(bblock_domain.end(), (g->n_bc + 255u) / 256u, (uint32_t)d);
+      // the fused order: every grid's own interleaving, grids in launch order
+      if (g->fused_host.empty()) {
+        const uint32_t nbk = (uint32_t)((g->info.cellCount + 255) / 256);
+        for (uint32_t k = 0; k < nbk; ++k) fused.push_back({(uint32_t)d, {k, FUSED_BULK}, 0u});
+      } else {
+        for (const FusedEntry& x : g->fused_host) fused.push_back({(uint32_t)d, x, 0u});
+      }
+    }
+    G.nbblk = (uint32_t)bblock_domain.size() - G.bblk0;
+    G.nfused = (uint32_t)fused.size() - G.fused0;
+    b->groups.push_back(G);
+    at0 = end;
   }
   for (int d = 0; d < nd; ++d) {
     const psl_grid* g = b->grids[d];
@@ -352,16 +465,23 @@ int build_batch(psl_batch* b) {
     b->total_bnd += g->n_bc;
     b->total_cells += g->info.cellCount;
   }
+  b->whole = BatchGroup{};
+  b->whole.ndom = (uint32_t)nd;
+  b->whole.ntile = (uint32_t)block_domain.size();
+  b->whole.nbblk = (uint32_t)bblock_domain.size();
+  b->whole.nfused = (uint32_t)fused.size();
   b->total_blocks = (uint32_t)block_domain.size();
   b->total_bblocks = (uint32_t)bblock_domain.size();
   b->total_fused = (uint32_t)fused.size();
   b->h_params = params;
   b->h_bparams = bparams;
   b->h_fbase = fbase;
+  params.insert(params.end(), params.begin(), params.begin() + nd);  // the two tables
   int rc = upload(&b->d_params, params);
   if (!rc) rc = upload(&b->d_bparams, bparams);
   if (!rc) rc = upload(&b->d_fbase, fbase);
   if (!rc) rc = upload(&b->d_delta, delta);
+  if (!rc) rc = upload(&b->d_dom, dom);
   if (!rc) rc = upload(&b->d_block_domain, block_domain);
   if (!rc) rc = upload(&b->d_block_tile, block_tile);
   if (!rc) rc = upload(&b->d_bblock_domain, bblock_domain);
@@ -466,6 +586,18 @@ int psl_batch_step(psl_batch* b, int nsteps) {
   }
   int rc = upload_shifts(b);
   if (rc) return rc;
+  // a batch beyond the cache: every group of grids runs all its steps in turn,
+  // launched as they are (a group's launches are long enough to hide their own
+  // enqueueing); one step of everything gains nothing from groups
+  if (nsteps > 1 && b->groups.size() > 1) {
+    for (const BatchGroup& G : b->groups) {
+      rc = enqueue_run(b, G, nsteps);
+      if (rc) return rc;
+    }
+    for (psl_grid* g : b->grids)
+      for (int s = 0; s < nsteps; ++s) psl_apply_streaming(g);
+    return PSL_OK;
+  }
   // whole graphs of steps_per_graph steps, then single steps
   const int k = b->steps_per_graph;
   if (k > 1 && nsteps >= k && !b->exec_k) {
