@@ -81,12 +81,17 @@ __global__ __launch_bounds__(64) void k_ps_boundary_staged(StagedParams p) {
                     });
 }
 
+// What the bulk launch does with the box-face cells: none listed, staged for
+// the boundary kernel, or updated in place (listed_mode).
+enum : int { LIST_NONE = 0, LIST_STAGE = 1, LIST_INLINE = 2 };
+
 // (held at the plain kernel's 7 waves per SIMD: without the bound the staging
 // branch raises the register count to 5 waves)
-template <class St, bool FLAGS, bool LES, int TUNE, bool STAGE, bool HELD = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_ps_bulk(StepParams p, Stage sg) {
-  bulk_update<St, FLAGS, LES, TUNE, STAGE, HELD>(p, p.xcd_remap ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x,
-                                                 sg);
+template <class St, bool FLAGS, bool LES, int TUNE, int LIST, bool HELD, bool COPY>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_ps_bulk(StepParams p, Stage sg,
+                                                                                         Faces fc, CopyStep cstep) {
+  bulk_update<St, FLAGS, LES, TUNE, LIST == LIST_STAGE, HELD, COPY, LIST == LIST_INLINE>(
+      p, p.xcd_remap ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x, sg, fc, cstep);
 }
 
 // Bulk cells with the learned closure in place of the Smagorinsky rate.
@@ -512,23 +517,45 @@ static void drop_profile_events(psl_grid* g) {
   g->prof_events.clear();
 }
 
-template <class St, int TUNE>
-static void launch_bulk(bool flags, bool les, bool held, uint32_t nb, size_t lds, hipStream_t stream,
-                        const StepParams& p, const Stage& sg) {
+// The bulk launch.  Non-temporal variants exist for the plain step only (not
+// with copies through the ring, box-face cells in place or a held closure).
+template <class St>
+static void launch_bulk(int nt, bool flags, bool les, bool held, int list, bool copy, uint32_t nb, size_t lds,
+                        hipStream_t stream, const StepParams& p, const Stage& sg, const Faces& fc,
+                        const CopyStep& cs) {
+#define PSL_BULK(F, L, V, M, H, C) k_ps_bulk<St, F, L, V, M, H, C><<<nb, 256, lds, stream>>>(p, sg, fc, cs)
+#define PSL_BULK_LES(F, V, M, C)                  \
+  do {                                            \
+    if (les) PSL_BULK(F, true, V, M, false, C);   \
+    else PSL_BULK(F, false, V, M, false, C);      \
+  } while (0)
   if (held) {
-    // between learned-closure evaluations (never staged)
-    if (flags) k_ps_bulk<St, true, true, TUNE, false, true><<<nb, 256, lds, stream>>>(p, sg);
-    else k_ps_bulk<St, false, true, TUNE, false, true><<<nb, 256, lds, stream>>>(p, sg);
-  } else if (sg.buf) {
-    if (les) k_ps_bulk<St, true, true, TUNE, true><<<nb, 256, lds, stream>>>(p, sg);
-    else k_ps_bulk<St, true, false, TUNE, true><<<nb, 256, lds, stream>>>(p, sg);
-  } else if (flags) {
-    if (les) k_ps_bulk<St, true, true, TUNE, false><<<nb, 256, lds, stream>>>(p, sg);
-    else k_ps_bulk<St, true, false, TUNE, false><<<nb, 256, lds, stream>>>(p, sg);
+    // between learned-closure evaluations
+    if (list == LIST_STAGE) PSL_BULK(true, true, 0, LIST_STAGE, true, false);
+    else if (flags) PSL_BULK(true, true, 0, LIST_NONE, true, false);
+    else PSL_BULK(false, true, 0, LIST_NONE, true, false);
+  } else if (list == LIST_INLINE) {
+    PSL_BULK_LES(true, 0, LIST_INLINE, false);
+  } else if (copy) {
+    if (flags) PSL_BULK_LES(true, 0, LIST_NONE, true);
+    else PSL_BULK_LES(false, 0, LIST_NONE, true);
   } else {
-    if (les) k_ps_bulk<St, false, true, TUNE, false><<<nb, 256, lds, stream>>>(p, sg);
-    else k_ps_bulk<St, false, false, TUNE, false><<<nb, 256, lds, stream>>>(p, sg);
+#define PSL_BULK_V(V)                                            \
+  case V:                                                        \
+    if (list == LIST_STAGE) PSL_BULK_LES(true, V, LIST_STAGE, false); \
+    else if (flags) PSL_BULK_LES(true, V, LIST_NONE, false);     \
+    else PSL_BULK_LES(false, V, LIST_NONE, false);               \
+    break
+    switch (nt) {
+      PSL_BULK_V(0);
+      PSL_BULK_V(1);
+      PSL_BULK_V(2);
+      PSL_BULK_V(3);
+    }
+#undef PSL_BULK_V
   }
+#undef PSL_BULK_LES
+#undef PSL_BULK
 }
 
 template <class St, int TUNE>
@@ -545,8 +572,40 @@ static void launch_fused(bool les, uint32_t nb, hipStream_t stream, const StepPa
   else k_ps_fused<St, false, TUNE><<<nb, 256, 0, stream>>>(p, b, order);
 }
 
+// Where the listed box-face cells are updated when they are not fused: in
+// place, each in its own lane of the bulk kernel, or staged for a launch of
+// their own.
+//
+// An x face is one cell per row.  In place, every wave that holds such a cell
+// runs restore + MBBC (and, for the 16-bit storages, a collision) for that one
+// lane, which costs VALU time; staged, a second launch stores 27 partial lines
+// per cell, which it must fetch again where the grid has left the last-level
+// cache, after a latency of about 10 us.  us per step of the sphere channel,
+// staged against in place: FP32, where the memory leaves the VALU idle,
+// 128x64x64 30.8 / 25.7, 256x128x128 213 / 198, 320x160x160 472 / 388; FP16
+// 128x64x64 27.3 / 24.8, 192x96x96 (91 MB) 49.9 / 51.7, 256x128x128 (216 MB)
+// 91 / 95, 320x160x160 (421 MB) 245 / 227; BF16 26 / 23, 49.8 / 48.4, 92 / 106,
+// 246 / 223, 203x97x121 (123 MB) 62 / 66.  So the 16-bit grids between the
+// latency-bound ones and those beyond the cache are staged.
+static int listed_mode(const psl_grid* g) {
+  const size_t bytes = 27ull * ncells(g) * storage_bytes(g->storage);
+  if (g->storage == PSL_F32) return LIST_INLINE;
+  return bytes < ((size_t)64 << 20) || bytes > ((size_t)256 << 20) ? LIST_INLINE : LIST_STAGE;
+}
+
+static Faces faces_of(const psl_grid* g) {
+  Faces f;
+  f.x = (g->periodic_copies & 1) && g->info.cellCountX > 1 ? g->ring_x : nullptr;
+  f.y = (g->periodic_copies & 2) && g->info.cellCountY > 1 ? g->ring_y : nullptr;
+  f.nx = make_fast_div((uint32_t)g->info.cellCountX);
+  f.ny = make_fast_div((uint32_t)g->info.cellCountY);
+  f.nz = (uint32_t)g->info.cellCountZ;
+  f.bc = g->bc_dev;
+  return f;
+}
+
 template <class St>
-static int launch_local_update(psl_grid* g, bool dominant_only = false) {
+static int launch_local_update(psl_grid* g, bool dominant_only = false, const CopyStep& cstep = CopyStep{}) {
   typedef typename St::T T;
   StepParams p;
   p.n = ncells(g);
@@ -599,6 +658,10 @@ static int launch_local_update(psl_grid* g, bool dominant_only = false) {
   }
   const int nt = g->tuning & (TUNE_NT_LOAD | TUNE_NT_STORE);
   const uint32_t nb = blocks_for(p.n);
+  // the network's own kernel updates them from their slots, held steps always stage them
+  const int list = !b.n || net || fused ? LIST_NONE : held ? LIST_STAGE : listed_mode(g);
+  const bool copy = cstep.in || cstep.out;
+  const Faces fc = faces_of(g);
   if (net) {
     const bool fl = g->flags != nullptr;
     const float nu = g->info.nu;
@@ -617,25 +680,16 @@ static int launch_local_update(psl_grid* g, bool dominant_only = false) {
       default: launch_fused<St, 3>(les, nf, g->stream, p, b, g->fused_dev); break;
     }
   } else {
-    const bool fl = g->flags != nullptr;
-    // the listed cells are staged by the bulk kernel whenever there are any
-    // (not between closure evaluations: the closure path updates them from
-    // their slots)
-    const Stage sg{b.n && !held ? g->stage_buf : nullptr, g->stage_base};
-    switch (nt) {
-      case 0: launch_bulk<St, 0>(fl, les, held, nb, g->bulk_lds, g->stream, p, sg); break;
-      case 1: launch_bulk<St, 1>(fl, les, held, nb, g->bulk_lds, g->stream, p, sg); break;
-      case 2: launch_bulk<St, 2>(fl, les, held, nb, g->bulk_lds, g->stream, p, sg); break;
-      default: launch_bulk<St, 3>(fl, les, held, nb, g->bulk_lds, g->stream, p, sg); break;
-    }
+    launch_bulk<St>(nt, g->flags != nullptr, les, held, list, copy, nb, g->bulk_lds, g->stream, p,
+                    Stage{list == LIST_STAGE ? g->stage_buf : nullptr, g->stage_base}, fc, cstep);
   }
   PSL_LAUNCH_CHECK();
   if (g->profile) {
     PSL_HIP_TRY(hipEventRecord(ev1, g->stream));
     g->prof_events.emplace_back(ev0, ev1);
   }
-  if (b.n && !fused && !dominant_only) {
-    if (net || held) k_ps_boundary<St><<<blocks_for(b.n), 256, 0, g->stream>>>(p, b);
+  if (b.n && !fused && !dominant_only && list != LIST_INLINE) {
+    if (net) k_ps_boundary<St><<<blocks_for(b.n), 256, 0, g->stream>>>(p, b);
     else {
       StagedParams sp;
       sp.f = g->f;
@@ -670,6 +724,9 @@ static int dispatch_storage(int storage, A... args) {
 }
 
 template <class St> struct LocalUpdateFn { static int run(psl_grid* g) { return launch_local_update<St>(g); } };
+template <class St> struct StepFn {
+  static int run(psl_grid* g, CopyStep c) { return launch_local_update<St>(g, false, c); }
+};
 template <class St> struct DominantFn { static int run(psl_grid* g) { return launch_local_update<St>(g, true); } };
 
 template <class St> struct FillEqFn {
@@ -726,6 +783,64 @@ static int periodic_copy(psl_grid* g, int axis) {
     k_periodic<uint16_t><<<grid, 256, 0, g->stream>>>((uint16_t*)g->f, shift_of(g), ncells(g), I.cellCountX,
                                                       I.cellCountY, row_blocks, axis);
   PSL_LAUNCH_CHECK();
+  return PSL_OK;
+}
+
+// Whether a call's steps pass the periodic copies on through the ring: the
+// rings exist, every cell is updated (a skipped cell leaves what it holds in
+// its slots, which only a copy pass sees) and the x faces are copied.  An x
+// copy moves one word per line (70 us per step on FP16 257x257x256, 2-4 us and
+// a launch on small grids), and through the ring costs the update 4 %; y
+// copies alone are contiguous passes of 5-10 us, no more than what the ring
+// costs the update (sphere channel 256x128x128 FP32: 198.8 us per step with
+// passes, 198.7 with the ring; 320x160x160 388 / 394).  Listed cells and the
+// learned closure keep the passes: their kernels have no registers to spare
+// (22 VGPR spills with the ring).
+static bool ring_runs(const psl_grid* g) {
+  return g->ring_x && !g->census[2] && !g->closure && !(g->flags && g->n_bc);
+}
+
+// The rings of the grid's copied faces, made when a call first has two steps;
+// without them (no memory, or a capture going on) the steps use copy passes.
+static void ensure_rings(psl_grid* g) {
+  const psl_info& I = g->info;
+  const size_t esz = storage_bytes(g->storage);
+  auto make = [&](void** p, size_t bytes) {
+    if (*p) return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(g->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+        hipMalloc(p, bytes) == hipSuccess)
+      return true;
+    *p = nullptr;
+    (void)hipGetLastError();
+    return false;
+  };
+  const bool y = (g->periodic_copies & 2) && I.cellCountY > 1;
+  if (y && !make(&g->ring_y, 4 * 9 * (size_t)I.cellCountX * I.cellCountZ * esz)) return;
+  (void)make(&g->ring_x, 4 * (size_t)I.cellCountY * I.cellCountZ * X_RUN * esz);
+}
+
+int grid_steps(psl_grid* g, int steps) {
+  bool ring = false;
+  if (steps > 1 && (g->periodic_copies & 1) && g->info.cellCountX > 1) {
+    ensure_rings(g);
+    ring = ring_runs(g);
+    // y copies of more than a layer need their ring too
+    if ((g->periodic_copies & 2) && g->info.cellCountY > 1 && !g->ring_y) ring = false;
+  }
+  CopyStep c{0u, false, false};
+  for (int s = 0; s < steps; ++s) {
+    int rc = psl_apply_streaming(g);
+    c.in = c.out;
+    c.half_in ^= 1u;
+    c.out = ring && s + 1 < steps;
+    if (!c.in) {
+      if (!rc && (g->periodic_copies & 1)) rc = psl_apply_bc_periodic_x(g);
+      if (!rc && (g->periodic_copies & 2)) rc = psl_apply_bc_periodic_y(g);
+    }
+    if (!rc) rc = dispatch_storage<StepFn>(g->storage, g, c);
+    if (rc) return rc;
+  }
   return PSL_OK;
 }
 
@@ -799,6 +914,8 @@ int psl_grid_destroy(psl_grid* g) {
   if (g->closure_y) (void)hipFree(g->closure_y);
   if (g->result) (void)hipFree(g->result);
   if (g->bc_dev) (void)hipFree(g->bc_dev);
+  if (g->ring_x) (void)hipFree(g->ring_x);
+  if (g->ring_y) (void)hipFree(g->ring_y);
   if (g->scalar_T) (void)hipFree(g->scalar_T);
   if (g->scalar_given) (void)hipFree(g->scalar_given);
   delete g;
@@ -1318,22 +1435,15 @@ int psl_grid_autotune(psl_grid* g, int steps, int* best, double* times_ms) {
   PSL_HIP_TRY(hipEventCreate(&e0));
   PSL_HIP_TRY(hipEventCreate(&e1));
   int rc = psl_grid_set_occupancy(g, 0);
-  // one whole step (streaming, periodic copies, local update): timed with the
-  // streaming, the rows are misaligned as in a run (repeated updates at one
-  // shift keep them where they are, at zero shift all line-aligned, where
-  // the non-temporal variants win and lose by a third once the rows move)
-  auto step = [&]() {
-    int r = psl_apply_streaming(g);
-    if (r == PSL_OK && (g->periodic_copies & 1)) r = psl_apply_bc_periodic_x(g);
-    if (r == PSL_OK && (g->periodic_copies & 2)) r = psl_apply_bc_periodic_y(g);
-    if (r == PSL_OK) r = psl_apply_local_cell_update(g);
-    return r;
-  };
+  // whole steps as a call of several runs them: timed with the streaming, the
+  // rows are misaligned as in a run (repeated updates at one shift keep them
+  // where they are, at zero shift all line-aligned, where the non-temporal
+  // variants win and lose by a third once the rows move)
   // mean ms of `n` steps after one warm-up, at the current settings
   auto time_updates = [&](double& mean, int n) {
-    int r = step();
+    int r = grid_steps(g, 1);
     if (r == PSL_OK && hipEventRecord(e0, g->stream) != hipSuccess) r = PSL_E_HIP;
-    for (int s = 0; s < n && r == PSL_OK; ++s) r = step();
+    if (r == PSL_OK) r = grid_steps(g, n);
     if (r == PSL_OK && hipEventRecord(e1, g->stream) != hipSuccess) r = PSL_E_HIP;
     float ms = 0.f;
     if (r == PSL_OK && (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess))

@@ -128,6 +128,8 @@ struct psl_grid {
   int closure_every = 1;          // network evaluated every closure_every local updates
   uint64_t closure_count = 0;     // local updates since the closure was set
   uint16_t* closure_y = nullptr;  // held network output per cell (FP16 bits), closure_every > 1
+  void* ring_x = nullptr;         // copied populations between two steps of a call, x faces (psl_stream.h)
+  void* ring_y = nullptr;         // the same, y faces
   float* scalar_T = nullptr;      // scalar-transport populations (27 * N FP32, same layout as f)
   float* scalar_given = nullptr;  // prescribed scalar per cell (NaN: free), or null
   float tau_t = 1.f;              // scalar relaxation time
@@ -260,6 +262,9 @@ int diad_macro_device(psl_diad* d, float* out4n);
 // implemented in psl_scalar.hip: the scalar value of every cell (n floats,
 // device) on the grid's stream
 int scalar_field_device(psl_grid* g, float* out);
+// implemented in psl_grid.hip: whole steps of one grid (streaming, periodic
+// copies, local update)
+int grid_steps(psl_grid* g, int steps);
 // implemented in psl_grid.hip
 int grid_rebuild_flags(psl_grid* g);
 int ensure_partials(psl_grid* g, size_t n);

@@ -382,15 +382,13 @@ static int comm_dispatch(psl_grid* c, psl_grid* f, bool full) {
 }
 
 static int update_level(psl_grid* const* levels, int nlevels, int level) {
-  psl_grid* g = levels[level];
-  int rc = psl_apply_streaming(g);
-  if (!rc && (g->periodic_copies & 1)) rc = psl_apply_bc_periodic_x(g);
-  if (!rc && (g->periodic_copies & 2)) rc = psl_apply_bc_periodic_y(g);
-  if (!rc) rc = psl_apply_local_cell_update(g);
+  int rc = grid_steps(levels[level], 1);
   if (rc) return rc;
   if (level < nlevels - 1) {
-    for (int i = 0; i < 2; ++i) {
-      rc = update_level(levels, nlevels, level + 1);
+    // the finest level's two steps have nothing between them
+    const int calls = level + 2 == nlevels ? 1 : 2;
+    for (int i = 0; i < calls; ++i) {
+      rc = calls == 1 ? grid_steps(levels[level + 1], 2) : update_level(levels, nlevels, level + 1);
       if (rc) return rc;
     }
     rc = comm_dispatch(levels[level], levels[level + 1], false);
@@ -416,6 +414,7 @@ int psl_update_grid(psl_grid* const* levels, int nlevels, int nsteps) {
     const int rc = comm_check(levels[l], levels[l + 1]);
     if (rc) return rc;
   }
+  if (nlevels == 1) return grid_steps(levels[0], nsteps);
   for (int s = 0; s < nsteps; ++s) {
     const int rc = update_level(levels, nlevels, 0);
     if (rc) return rc;

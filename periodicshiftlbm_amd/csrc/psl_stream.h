@@ -364,13 +364,180 @@ __device__ __forceinline__ void load_staged(const float* stage, uint32_t t, floa
   fl = (int)__builtin_bit_cast(uint32_t, wf);
 }
 
+// ------------------------------------------------- periodic copies in the step
+// applyBCPeriodicX/Y (include/boundaryConditions/periodicXY.h:38-128) between
+// two steps of one call, without a pass of its own.  After streaming, a copy
+// replaces population q of a face cell by that of the cell across (+c right to
+// left, -c left to right; x before y).  The value copied is the one the step
+// before stored in the across cell's slot, so that step also writes it into a
+// ring buffer (copy_out), and the face cell's update reads it from there
+// instead of from its slot (copy_in).  Reading the across cell's slot itself
+// would race with that cell's update in the same launch; the two ring halves
+// are used by alternate steps, so no step reads what it writes.  Layout: x
+// faces 9 words per row (one lane's contiguous run, padded to 16), y faces one
+// row of words along i per population (consecutive lanes are consecutive i).
+struct FastDiv {  // x / d for x < 2^31
+  uint32_t d, m, s;
+};
+__host__ __device__ inline uint32_t fast_div(uint32_t x, const FastDiv& f) {
+  return f.s ? (uint32_t)(((uint64_t)x * f.m) >> 32) >> (f.s - 1u) : x;
+}
+inline FastDiv make_fast_div(uint32_t d) {
+  FastDiv f{d, 0u, 0u};
+  while ((1ull << f.s) < d) ++f.s;
+  f.m = f.s ? (uint32_t)((1ull << (31 + f.s)) / d + 1u) : 0u;
+  return f;
+}
+
+constexpr int X_RUN = 16;  // words per row of an x face's buffer
+struct Faces {
+  void* x;         // ring of the x copies: 2 halves x 2 sides x (ny nz) rows x X_RUN, or null: none
+  void* y;         // ring of the y copies: 2 halves x 2 sides x 9 x (nx nz), or null: none
+  FastDiv nx, ny;  // cells per row, rows per plane
+  uint32_t nz;
+  const float4* bc;  // given-value slots, for box-face cells updated in the bulk kernel
+};
+// The ring half a step reads (it writes the other), and whether it does either.
+struct CopyStep {
+  uint32_t half_in;
+  bool in, out;
+};
+
+constexpr int rank_of(const int (&c)[27], int q) {  // populations of the same sign of c below q
+  int r = 0;
+  for (int p = 0; p < q; ++p) r += c[p] == c[q];
+  return r;
+}
+
+// Position of a cell and whether its wave has any lane near a copied face
+// (face layers and, for the writers, the layers whose populations move there).
+struct CopyLane {
+  bool wave_near;
+  uint32_t i, j, k, row;
+};
+__device__ __forceinline__ CopyLane cell_position(const Faces& c, uint32_t cell) {
+  CopyLane l;
+  l.wave_near = true;
+  l.row = fast_div(cell, c.nx);
+  l.i = cell - l.row * c.nx.d;
+  l.k = fast_div(l.row, c.ny);
+  l.j = l.row - l.k * c.ny.d;
+  return l;
+}
+__device__ __forceinline__ CopyLane copy_lane(const Faces& c, uint32_t w_first, uint32_t cell) {
+  CopyLane l;
+  const uint32_t nx = c.nx.d, ny = c.ny.d;
+  const uint32_t row0 = fast_div(w_first, c.nx), i0 = w_first - row0 * nx;
+  const uint32_t rows = fast_div(w_first + 63u, c.nx) - row0;
+  const uint32_t j0 = row0 - fast_div(row0, c.ny) * ny;
+  const bool near = (c.x && (i0 < 2u || i0 + 65u >= nx)) || (c.y && (j0 < 3u || j0 + rows + 3u >= ny));
+  if (near) return cell_position(c, cell);
+  l.wave_near = false;
+  l.i = l.j = l.k = l.row = 0u;
+  return l;
+}
+
+template <class T>
+__device__ __forceinline__ T* ring_x(const Faces& c, uint32_t half, int cx) {
+  return (T*)c.x + (size_t)(2u * half + (cx > 0 ? 1u : 0u)) * c.ny.d * c.nz * X_RUN;
+}
+template <class T>
+__device__ __forceinline__ T* ring_y(const Faces& c, uint32_t half, int cy, int q) {
+  return (T*)c.y + ((size_t)(2u * half + (cy > 0 ? 1u : 0u)) * 9u + rank_of(CY, q)) * ((size_t)c.nx.d * c.nz);
+}
+
+// The copied populations of a face cell, as storage words.
+template <class St>
+__device__ __forceinline__ void copy_in(const Faces& c, uint32_t half, const CopyLane& l, Word<St> (&r)[27]) {
+  typedef typename St::T T;
+  const uint32_t nx = c.nx.d, ny = c.ny.d;
+  const bool y0 = c.y && l.j == 0u, y1 = c.y && l.j == ny - 1u;
+  if (c.x && (l.i == 0u || l.i == nx - 1u)) {
+#pragma unroll
+    for (int q = 0; q < 27; ++q) {
+      if (CX[q] == 0) continue;
+      // across in y too where that copy applies
+      const uint32_t row = CY[q] > 0 && y0 ? l.row + (ny - 1u) : CY[q] < 0 && y1 ? l.row - (ny - 1u) : l.row;
+      if (l.i == (CX[q] > 0 ? 0u : nx - 1u))
+        r[q] = (Word<St>)ld<T, false>(ring_x<T>(c, half, CX[q]) + (size_t)row * X_RUN + rank_of(CX, q));
+    }
+  }
+  if (y0 || y1) {
+    const uint32_t at = l.k * nx + l.i;
+#pragma unroll
+    for (int q = 0; q < 27; ++q) {
+      if (CY[q] == 0) continue;
+      const bool by_x = CX[q] != 0 && c.x && l.i == (CX[q] > 0 ? 0u : nx - 1u);
+      if ((CY[q] > 0 ? y0 : y1) && !by_x) r[q] = (Word<St>)ld<T, false>(ring_y<T>(c, half, CY[q], q) + at);
+    }
+  }
+}
+
+// v modulo m for -2 m <= v < 3 m (a single row or plane wraps twice)
+__device__ __forceinline__ int wrapped(int v, int m) {
+  if (v < 0) v += m;
+  if (v < 0) v += m;
+  if (v >= m) v -= m;
+  if (v >= m) v -= m;
+  return v;
+}
+
+// What a cell's update leaves in slots that a face cell's copy will be taken
+// from: population q moves to the cell at linear index cell + d_q (rows and
+// planes run on into each other there, as the slots do).
+template <class St, class Get>
+__device__ __forceinline__ void copy_out(const Faces& c, uint32_t half, const CopyLane& l, Get&& word) {
+  typedef typename St::T T;
+  const uint32_t nx = c.nx.d, ny = c.ny.d, rows = ny * c.nz;
+  if (c.x && (l.i == 1u || l.i + 2u == nx)) {
+#pragma unroll
+    for (int q = 0; q < 27; ++q) {
+      if (CX[q] == 0) continue;
+      if (CX[q] > 0 ? l.i + 2u == nx : l.i == 1u) {
+        const int row = wrapped((int)l.row + CY[q] + (int)ny * CZ[q], (int)rows);
+        st<T, false>(ring_x<T>(c, half, CX[q]) + (size_t)row * X_RUN + rank_of(CX, q), word(q));
+      }
+    }
+  }
+  if (c.y && (l.j < 3u || l.j + 3u >= ny)) {
+#pragma unroll
+    for (int q = 0; q < 27; ++q) {
+      if (CY[q] == 0) continue;
+      int i = (int)l.i + CX[q], j = (int)l.j + CY[q], k = (int)l.k + CZ[q];
+      if (CX[q] < 0 && i < 0) {
+        i += (int)nx;
+        --j;
+      }
+      if (CX[q] > 0 && i >= (int)nx) {
+        i -= (int)nx;
+        ++j;
+      }
+      if (j < 0) {
+        j += (int)ny;
+        --k;
+      }
+      if (j >= (int)ny) {
+        j -= (int)ny;
+        ++k;
+      }
+      k = wrapped(k, (int)c.nz);
+      if (j == (CY[q] > 0 ? (int)ny - 1 : 0))
+        st<T, false>(ring_y<T>(c, half, CY[q], q) + (size_t)k * nx + i, word(q));
+    }
+  }
+}
+
 // Fluid and bounceback cells of one block in cell order; with STAGE the
 // listed box-face cells of the block are loaded too and written to their
 // staging records (their update is the boundary kernel's).  HELD: a step
 // between evaluations of a learned closure, relaxing with the network output
-// stored per cell (p.nut_y) and no Smagorinsky term.
-template <class St, bool FLAGS, bool LES, int TUNE, bool STAGE = false, bool HELD = false>
-__device__ __forceinline__ void bulk_update(const StepParams& p, uint32_t block, const Stage& sg = Stage{}) {
+// stored per cell (p.nut_y) and no Smagorinsky term.  COPY: the periodic
+// copies come and go through the ring (cr, cstep).  INL: the listed cells are
+// updated here, each in its own lane.
+template <class St, bool FLAGS, bool LES, int TUNE, bool STAGE = false, bool HELD = false, bool COPY = false,
+          bool INL = false>
+__device__ __forceinline__ void bulk_update(const StepParams& p, uint32_t block, const Stage& sg = Stage{},
+                                            const Faces& cr = Faces{}, const CopyStep& cstep = CopyStep{}) {
   const uint32_t block_first = block * 256u;
   const uint32_t cell = block_first + threadIdx.x;
   const uint32_t w_first = wave_first_cell(block_first);
@@ -381,13 +548,24 @@ __device__ __forceinline__ void bulk_update(const StepParams& p, uint32_t block,
   int fl = 0;
   if (FLAGS) fl = ld<uint8_t, false>(p.flags + cell);
   const int kind = FLAGS ? fl & 7 : KIND_FLUID;
-  if (kind > (STAGE ? KIND_GIVEN_RHOU : KIND_BOUNCEBACK)) return;
+  if (kind > (STAGE || INL ? KIND_GIVEN_RHOU : KIND_BOUNCEBACK)) return;
   // the stored network output is loaded ahead of the populations, so that it
   // is in flight with them rather than after them
   uint16_t y_held = 0;
   if constexpr (HELD) y_held = ld<uint16_t, false>(p.nut_y + cell);
   Word<St> r[27];
   load27_raw<St, TUNE>(p, w_first, straddle, cell, r);
+  CopyLane cl;
+  if constexpr (COPY) {
+    cl = copy_lane(cr, w_first, cell);
+    if (cstep.in && cl.wave_near) {
+      copy_in<St>(cr, cstep.half_in, cl, r);
+      // as in load27_raw: the words leave the branch as 32-bit values
+      __asm__ volatile("" ::: "memory");
+#pragma unroll
+      for (int q = 0; q < 27; ++q) __asm__("" : "+v"(r[q]));
+    }
+  }
   float v[27];
   if (STAGE) {
     const bool listed = kind >= KIND_GIVEN_RHO;
@@ -415,7 +593,32 @@ __device__ __forceinline__ void bulk_update(const StepParams& p, uint32_t block,
       }
     }
   }
-  if (kind == KIND_BOUNCEBACK) {
+  if (INL && kind >= KIND_GIVEN_RHO) {
+    // box-face cell in place: restore + MBBC (boundary_core) on the loaded words
+    words_to_float<St>(r, v);
+    if (St::W_OFF) {
+#pragma unroll
+      for (int q = 0; q < 27; ++q) v[q] += weight(q);
+    }
+    const CopyLane at = cell_position(cr, cell);
+    const float* g = (const float*)(cr.bc + ((fl >> 6) & 3));
+    boundary_cell(v, kind, outer_normal_code((int)at.i, (int)at.j, (int)at.k, (int)cr.nx.d, (int)cr.ny.d, (int)cr.nz, fl),
+                  ld<float, false>(g), ld<float, false>(g + 1), ld<float, false>(g + 2), ld<float, false>(g + 3));
+    if constexpr (!St::W_OFF) {
+      // FP32: on to the collision with the wave's other lanes
+#pragma unroll
+      for (int q = 0; q < 27; ++q) r[q] = v[q];
+    } else {
+      // 16-bit storage: the collision on full f, as the staged path's
+      const float cs = p.cs_cell ? ld<float, false>(p.cs_cell + cell) : p.cs;
+      collide<false>(v, Relax{p.omega, p.tau, p.cs}, cs);
+#pragma unroll
+      for (int q = 0; q < 27; ++q) v[q] -= weight(q);
+    }
+  }
+  if (INL && St::W_OFF && kind >= KIND_GIVEN_RHO) {
+    // done
+  } else if (kind == KIND_BOUNCEBACK) {
     // the swap commutes with "f - w" (opposite directions share a weight)
     words_to_float<St>(r, v);
     bounceback(v);
@@ -432,6 +635,10 @@ __device__ __forceinline__ void bulk_update(const StepParams& p, uint32_t block,
     collide_with_moments<St::W_OFF>(v, raw_moments_words<St>(r), rx, LES ? cs : 0.f);
   }
   store27<St, TUNE>(p, w_first, straddle, cell, v);
+  if constexpr (COPY) {
+    if (cstep.out && cl.wave_near)
+      copy_out<St>(cr, cstep.half_in ^ 1u, cl, [&](int q) { return St::store(v[q]); });
+  }
 }
 
 }  // namespace psl

@@ -1,0 +1,71 @@
+"""Calls of several steps (psl_update_grid) against the same steps one call at a
+time: the periodic copies passed on inside the update, and the box-face cells
+updated in the bulk kernel or staged, leave the same bits in every cell."""
+import numpy as np
+import pytest
+
+from periodicshiftlbm_amd import cases
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(P, shape, storage, copies, seed, flags=None):
+    rng = np.random.default_rng(seed)
+    nx, ny, nz = shape
+    n = nx * ny * nz
+    g = P.GridStruct(P.InfoStruct(cellCountX=nx, cellCountY=ny, cellCountZ=nz, nu=0.01), storage)
+    if flags is not None:
+        g.set_flags(flags)
+        g.set_given_values(cases.channel_given_values(0.03))
+    g.set_smagorinsky(0.12 if seed % 2 else 0.0)
+    g.set_periodic_copies(x=copies[0], y=copies[1])
+    P.fill_equilibrium(g, rng.uniform(0.98, 1.02, n).astype(np.float32),
+                       *rng.uniform(-0.03, 0.03, (3, n)).astype(np.float32))
+    return g
+
+
+def _same(a, b, what):
+    assert a.shifter.tolist() == b.shifter.tolist()
+    nbad = int(np.count_nonzero(a.get_f().view(np.uint32) != b.get_f().view(np.uint32)))
+    assert nbad == 0, f"{what}: {nbad} values differ"
+
+
+# rows shorter than, equal to and longer than a wave and a workgroup; single and
+# double layers on every axis, where a copied face is its own or its neighbour's
+SHAPES = [(2, 2, 1), (2, 1, 3), (3, 2, 2), (5, 1, 1), (17, 17, 16), (63, 3, 2), (64, 4, 3), (65, 5, 1), (130, 2, 3),
+          (257, 9, 4), (300, 1, 2)]
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("copies", [(True, False), (True, True)])
+def test_copies_inside_a_call_equal_copy_passes(psl, storage, copies):
+    P = psl
+    for s, shape in enumerate(SHAPES):
+        n = shape[0] * shape[1] * shape[2]
+        solid = None
+        if s % 3 == 2:  # bounceback cells, on the copied faces too
+            solid = np.where(np.random.default_rng(s).random(n) < 0.2, cases.BOUNCEBACK, cases.FLUID).astype(np.uint8)
+        a, b = (_grid(P, shape, storage, copies, s, solid) for _ in range(2))
+        for steps in (2, 5):
+            P.updateGrid([a], steps)
+            for _ in range(steps):
+                P.updateGrid([b], 1)
+            _same(a, b, f"{shape} after {steps}")
+        a.close()
+        b.close()
+
+
+# FP16 / BF16: 69 MB is staged; 21 MB and 286 MB, and every FP32 grid, are updated in place
+@pytest.mark.parametrize("storage,shape", [("f16", (128, 100, 100)), ("bf16", (130, 99, 101)), ("f16", (74, 73, 72)),
+                                           ("f16", (260, 145, 141)), ("f32", (131, 70, 69))])
+def test_box_faces_staged_and_in_place_equal_the_fused_launch(psl, storage, shape):
+    P = psl
+    rng = np.random.default_rng(3)
+    flags = cases.channel_flags(shape, rng.random(shape[0] * shape[1] * shape[2]) < 0.02)
+    a, b = (_grid(P, shape, storage, (False, True), 3, flags) for _ in range(2))
+    b.tuning = P.TUNE_FUSED_BOUNDARY
+    P.updateGrid([a], 3)
+    P.updateGrid([b], 3)
+    _same(a, b, f"{storage} {shape}")
+    a.close()
+    b.close()
