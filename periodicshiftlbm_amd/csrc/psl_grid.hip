@@ -796,6 +796,10 @@ static int periodic_copy(psl_grid* g, int axis) {
 // passes, 198.7 with the ring; 320x160x160 388 / 394).  Listed cells and the
 // learned closure keep the passes: their kernels have no registers to spare
 // (22 VGPR spills with the ring).
+// Grids under RING_CELLS keep them too: their step is bound by latency, most of
+// it fetching the kernels' instructions (us per step, passes against ring: FP16
+// 17x17x16 12.4 / 13.7, 33x33x32 12.9 / 12.4, 65x65x64 19.2 / 15.3).
+constexpr uint32_t RING_CELLS = 32768;
 static bool ring_runs(const psl_grid* g) {
   return g->ring_x && !g->census[2] && !g->closure && !(g->flags && g->n_bc);
 }
@@ -822,7 +826,7 @@ static void ensure_rings(psl_grid* g) {
 
 int grid_steps(psl_grid* g, int steps) {
   bool ring = false;
-  if (steps > 1 && (g->periodic_copies & 1) && g->info.cellCountX > 1) {
+  if (steps > 1 && (g->periodic_copies & 1) && g->info.cellCountX > 1 && ncells(g) >= RING_CELLS) {
     ensure_rings(g);
     ring = ring_runs(g);
     // y copies of more than a layer need their ring too

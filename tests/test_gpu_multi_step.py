@@ -30,10 +30,11 @@ def _same(a, b, what):
     assert nbad == 0, f"{what}: {nbad} values differ"
 
 
-# rows shorter than, equal to and longer than a wave and a workgroup; single and
-# double layers on every axis, where a copied face is its own or its neighbour's
-SHAPES = [(2, 2, 1), (2, 1, 3), (3, 2, 2), (5, 1, 1), (17, 17, 16), (63, 3, 2), (64, 4, 3), (65, 5, 1), (130, 2, 3),
-          (257, 9, 4), (300, 1, 2)]
+# (from 32768 cells on) rows shorter than, equal to and longer than a wave and a
+# workgroup; single and double layers on every axis, where a copied face is its
+# own or its neighbour's
+SHAPES = [(2, 130, 128), (3, 200, 60), (5, 100, 70), (17, 50, 41), (63, 3, 180), (64, 4, 130), (65, 5, 110),
+          (130, 2, 130), (257, 9, 15), (300, 1, 112), (2, 1, 20000), (17000, 2, 1), (40000, 1, 1)]
 
 
 @pytest.mark.parametrize("storage", ["f32", "f16", "bf16"])
