@@ -13,9 +13,9 @@
 //      Pi = -(2/3) rho tau_eff S with tau_eff = 3 (nu + nu_t*) + 1/2, and from
 //      them the raw closure inputs (closure_features);
 //   4. training: mean-squared error of y against nu_t* / NU_SCALE, Adam,
-//      mini-batches drawn by a counter-based generator; per-sample forward and
-//      backward in k_mlp_fwd_bwd, deterministic gradient reduction in
-//      k_mlp_grad_partial + k_mlp_adam (fixed summation order);
+//      mini-batches drawn by a counter-based generator; forward, backward and
+//      gradient sums of 64 rows per workgroup in k_mlp_batch, their total and
+//      the update in k_mlp_adam (fixed summation order);
 //   5. inference inside the step (closure_wave, psl_closure.h).
 #include "psl_closure.h"
 #include "psl_stream.h"
@@ -26,131 +26,199 @@
 namespace psl {
 
 // ------------------------------------------------------------ training
-struct TrainBufs {
-  float* h1;   // B x 32
-  float* h2;   // B x 32
-  float* dz1;  // B x 32
-  float* dz2;  // B x 32
-  float* dy;   // B
-  float* sq;   // B squared errors
-};
+// One iteration is two launches.  What bounds it is latency, not work (a
+// 16384-row batch is 0.13 GFLOP): with one row per thread and its 32-wide
+// layers in scratch the forward/backward pass took 42 us, the gradient pass
+// another 16 us over activations written to memory, and the update 59 us in
+// 256 serial additions per parameter, 125 us with the index launch.  Here a
+// workgroup takes 64 rows through both passes and their gradients in LDS and
+// the update adds the workgroups' sums 16 ways at once: 17 us per iteration.
+constexpr int CHUNK = 64;     // rows per workgroup
+constexpr int ROWS = 64 + 4;  // LDS row length: 16-byte aligned, rows 4 banks apart
 
-// Per-sample forward pass and deltas.  x: standardised inputs (n x 9) of the
-// whole set, idx: the batch (B indices into x), t: targets.
-__global__ __launch_bounds__(256) void k_mlp_fwd_bwd(const float* __restrict__ P, const float* __restrict__ x,
-                                                     const float* __restrict__ t, const uint32_t* __restrict__ idx,
-                                                     int B, TrainBufs tb) {
-  const int b = blockIdx.x * 256 + threadIdx.x;
-  if (b >= B) return;
-  const uint32_t s = idx ? idx[b] : (uint32_t)b;
+// The rows of a mini-batch: row b of iteration `step` is splitmix64(seed, step,
+// b) mod n, or b itself (draw = false).
+struct BatchDraw {
+  bool draw;
+  uint32_t n;
+  uint64_t recip;  // floor((2^64 - 1) / n)
+  uint64_t seed;
+  int step;
+};
+__device__ __forceinline__ uint32_t batch_row(const BatchDraw& d, int B, int b) {
+  if (!d.draw) return (uint32_t)b;
+  uint64_t z = d.seed + ((uint64_t)d.step * (uint64_t)B + (uint64_t)b + 1ull) * 0x9E3779B97F4A7C15ull;
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z ^= z >> 31;
+  // z mod n: the quotient from the reciprocal is at most two short
+  uint64_t r = z - __umul64hi(z, d.recip) * d.n;
+  if (r >= d.n) r -= d.n;
+  if (r >= d.n) r -= d.n;
+  return (uint32_t)r;
+}
+
+__device__ __forceinline__ float dot4(const float4& a, const float4& b, float s) {
+  s += a.x * b.x;
+  s += a.y * b.y;
+  s += a.z * b.z;
+  return s + a.w * b.w;
+}
+// sum over the workgroup's rows of a[row] b[row] (two LDS rows), in row order
+__device__ __forceinline__ float dot_rows(const float* a, const float* b) {
+  float s = 0.f;
+#pragma unroll
+  for (int r = 0; r < CHUNK; r += 4) s = dot4(*(const float4*)(a + r), *(const float4*)(b + r), s);
+  return s;
+}
+__device__ __forceinline__ float sum_rows(const float* a) {
+  float s = 0.f;
+#pragma unroll
+  for (int r = 0; r < CHUNK; ++r) s += a[r];
+  return s;
+}
+
+// Forward and backward pass of CHUNK rows and their gradient sums (fixed
+// order) into partial[block][MLP_PARAMS + 1], the squared error last.  Lane =
+// row, wave w = hidden units 8 w .. 8 w + 7 of each layer, so that the weights
+// are wave-uniform (scalar loads) and an LDS array [unit][row] is read without
+// bank conflicts in the passes and 16 bytes at a time in the gradient sums.
+__global__ __launch_bounds__(256) void k_mlp_batch(const float* __restrict__ P, const float* __restrict__ x,
+                                                   const float* __restrict__ t, BatchDraw draw, int B,
+                                                   float* __restrict__ partial) {
+  __shared__ __align__(16) float sx[MLP_IN][ROWS];
+  __shared__ __align__(16) float h1[MLP_HID][ROWS], h2[MLP_HID][ROWS], z1[MLP_HID][ROWS], z2[MLP_HID][ROWS];
+  __shared__ __align__(16) float sy[4][ROWS], sdy[ROWS], ssq[ROWS];
+  constexpr int U = MLP_HID / 4;  // units per wave
   const float* W1 = P;
   const float* b1 = W1 + MLP_IN * MLP_HID;
   const float* W2 = b1 + MLP_HID;
   const float* b2 = W2 + MLP_HID * MLP_HID;
   const float* W3 = b2 + MLP_HID;
-  const float b3 = W3[MLP_HID];
+  const int r = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), u0 = w * U;
+  const int b = blockIdx.x * CHUNK + r;
+  const bool live = b < B;  // rows past the batch repeat its last one with no error
+  const size_t row = batch_row(draw, B, live ? b : B - 1);
   float xi[MLP_IN];
 #pragma unroll
-  for (int i = 0; i < MLP_IN; ++i) xi[i] = x[(size_t)s * MLP_IN + i];
-  float h1[MLP_HID], h2[MLP_HID];
-  for (int h = 0; h < MLP_HID; ++h) {
-    float z = b1[h];
+  for (int i = 0; i < MLP_IN; ++i) xi[i] = x[row * MLP_IN + i];
+  const float target = t[row];
 #pragma unroll
-    for (int i = 0; i < MLP_IN; ++i) z += xi[i] * W1[i * MLP_HID + h];
-    h1[h] = tanhf(z);
+  for (int j = 0; j < U; ++j) {
+    float z = b1[u0 + j];
+#pragma unroll
+    for (int i = 0; i < MLP_IN; ++i) z += xi[i] * W1[i * MLP_HID + u0 + j];
+    h1[u0 + j][r] = tanhf(z);
   }
-  float y = b3;
-  for (int g = 0; g < MLP_HID; ++g) {
-    float z = b2[g];
-    for (int h = 0; h < MLP_HID; ++h) z += h1[h] * W2[h * MLP_HID + g];
-    h2[g] = tanhf(z);
-    y += h2[g] * W3[g];
+  if (w == 0) {
+#pragma unroll
+    for (int i = 0; i < MLP_IN; ++i) sx[i][r] = xi[i];
   }
-  const float e = y - t[s];
-  const float dy = 2.f * e / (float)B;
-  tb.dy[b] = dy;
-  tb.sq[b] = e * e;
-  float dz2[MLP_HID];
-  for (int g = 0; g < MLP_HID; ++g) {
-    dz2[g] = dy * W3[g] * (1.f - h2[g] * h2[g]);
-    tb.h1[(size_t)b * MLP_HID + g] = h1[g];
-    tb.h2[(size_t)b * MLP_HID + g] = h2[g];
-    tb.dz2[(size_t)b * MLP_HID + g] = dz2[g];
-  }
+  __syncthreads();
+  float z[U];
+#pragma unroll
+  for (int j = 0; j < U; ++j) z[j] = b2[u0 + j];
+#pragma unroll 8
   for (int h = 0; h < MLP_HID; ++h) {
-    float d = 0.f;
-    for (int g = 0; g < MLP_HID; ++g) d += dz2[g] * W2[h * MLP_HID + g];
-    tb.dz1[(size_t)b * MLP_HID + h] = d * (1.f - h1[h] * h1[h]);
+    const float a = h1[h][r];
+#pragma unroll
+    for (int j = 0; j < U; ++j) z[j] += a * W2[h * MLP_HID + u0 + j];
   }
-}
-
-// Partial gradient sums over a chunk of CHUNK samples per block (fixed order),
-// plus the partial squared error in slot MLP_PARAMS.
-constexpr int CHUNK = 64;
-__global__ __launch_bounds__(256) void k_mlp_grad_partial(const float* __restrict__ x,
-                                                          const uint32_t* __restrict__ idx, int B, TrainBufs tb,
-                                                          float* __restrict__ partial) {
-  __shared__ float sx[CHUNK][MLP_IN];
-  __shared__ float sh1[CHUNK][MLP_HID];
-  __shared__ float sh2[CHUNK][MLP_HID];
-  __shared__ float sz1[CHUNK][MLP_HID];
-  __shared__ float sz2[CHUNK][MLP_HID];
-  __shared__ float sdy[CHUNK];
-  __shared__ float ssq[CHUNK];
-  const int b0 = blockIdx.x * CHUNK;
-  const int nb = min(CHUNK, B - b0);
-  for (int e = threadIdx.x; e < CHUNK * MLP_HID; e += 256) {
-    const int r = e / MLP_HID, c = e % MLP_HID;
-    const bool ok = r < nb;
-    const size_t o = (size_t)(b0 + r) * MLP_HID + c;
-    sh1[r][c] = ok ? tb.h1[o] : 0.f;
-    sh2[r][c] = ok ? tb.h2[o] : 0.f;
-    sz1[r][c] = ok ? tb.dz1[o] : 0.f;
-    sz2[r][c] = ok ? tb.dz2[o] : 0.f;
+  float y = 0.f;
+#pragma unroll
+  for (int j = 0; j < U; ++j) {
+    z[j] = tanhf(z[j]);
+    h2[u0 + j][r] = z[j];
+    y += z[j] * W3[u0 + j];
   }
-  for (int e = threadIdx.x; e < CHUNK * MLP_IN; e += 256) {
-    const int r = e / MLP_IN, c = e % MLP_IN;
-    sx[r][c] = r < nb ? x[(size_t)(idx ? idx[b0 + r] : (uint32_t)(b0 + r)) * MLP_IN + c] : 0.f;
+  sy[w][r] = y;
+  __syncthreads();
+  const float err = live ? W3[MLP_HID] + ((sy[0][r] + sy[1][r]) + (sy[2][r] + sy[3][r])) - target : 0.f;
+  const float dy = 2.f * err / (float)B;
+  if (w == 0) {
+    sdy[r] = dy;
+    ssq[r] = err * err;
   }
-  for (int r = threadIdx.x; r < CHUNK; r += 256) {
-    sdy[r] = r < nb ? tb.dy[b0 + r] : 0.f;
-    ssq[r] = r < nb ? tb.sq[b0 + r] : 0.f;
+#pragma unroll
+  for (int j = 0; j < U; ++j) z2[u0 + j][r] = dy * W3[u0 + j] * (1.f - z[j] * z[j]);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < U; ++j) z[j] = 0.f;
+#pragma unroll 8
+  for (int g = 0; g < MLP_HID; ++g) {
+    const float d = z2[g][r];
+#pragma unroll
+    for (int j = 0; j < U; ++j) z[j] += d * W2[(u0 + j) * MLP_HID + g];
+  }
+#pragma unroll
+  for (int j = 0; j < U; ++j) {
+    const float a = h1[u0 + j][r];
+    z1[u0 + j][r] = z[j] * (1.f - a * a);
   }
   __syncthreads();
   float* out = partial + (size_t)blockIdx.x * (MLP_PARAMS + 1);
-  for (int p = threadIdx.x; p < MLP_PARAMS + 1; p += 256) {
-    float s = 0.f;
-    int q = p;
-    if (q < MLP_IN * MLP_HID) {  // W1[i][h]
-      const int i = q / MLP_HID, h = q % MLP_HID;
-      for (int r = 0; r < CHUNK; ++r) s += sx[r][i] * sz1[r][h];
-    } else if ((q -= MLP_IN * MLP_HID) < MLP_HID) {  // b1
-      for (int r = 0; r < CHUNK; ++r) s += sz1[r][q];
-    } else if ((q -= MLP_HID) < MLP_HID * MLP_HID) {  // W2[h][g]
-      const int h = q / MLP_HID, g = q % MLP_HID;
-      for (int r = 0; r < CHUNK; ++r) s += sh1[r][h] * sz2[r][g];
-    } else if ((q -= MLP_HID * MLP_HID) < MLP_HID) {  // b2
-      for (int r = 0; r < CHUNK; ++r) s += sz2[r][q];
-    } else if ((q -= MLP_HID) < MLP_HID) {  // W3
-      for (int r = 0; r < CHUNK; ++r) s += sh2[r][q] * sdy[r];
-    } else if (q == MLP_HID) {  // b3
-      for (int r = 0; r < CHUNK; ++r) s += sdy[r];
-    } else {  // squared error
-      for (int r = 0; r < CHUNK; ++r) s += ssq[r];
+  // W2[h][g], a 2 x 2 tile per thread
+  {
+    const int h = 2 * (threadIdx.x >> 4), g = 2 * (threadIdx.x & 15);
+    float s00 = 0.f, s01 = 0.f, s10 = 0.f, s11 = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < CHUNK; k += 4) {
+      const float4 a0 = *(const float4*)&h1[h][k], a1 = *(const float4*)&h1[h + 1][k];
+      const float4 c0 = *(const float4*)&z2[g][k], c1 = *(const float4*)&z2[g + 1][k];
+      s00 = dot4(a0, c0, s00);
+      s01 = dot4(a0, c1, s01);
+      s10 = dot4(a1, c0, s10);
+      s11 = dot4(a1, c1, s11);
     }
-    out[p] = s;
+    float* o = out + MLP_IN * MLP_HID + MLP_HID + h * MLP_HID + g;
+    o[0] = s00;
+    o[1] = s01;
+    o[MLP_HID] = s10;
+    o[MLP_HID + 1] = s11;
+  }
+  // W1[i][h], b1, b2, W3, b3, squared error
+  constexpr int REST = MLP_IN * MLP_HID + 3 * MLP_HID + 2;
+  for (int p = threadIdx.x; p < REST; p += 256) {
+    int q = p;
+    if (q < MLP_IN * MLP_HID) {
+      out[q] = dot_rows(sx[q / MLP_HID], z1[q % MLP_HID]);
+    } else if ((q -= MLP_IN * MLP_HID) < MLP_HID) {
+      out[MLP_IN * MLP_HID + q] = sum_rows(z1[q]);
+    } else if ((q -= MLP_HID) < MLP_HID) {
+      out[MLP_IN * MLP_HID + MLP_HID + MLP_HID * MLP_HID + q] = sum_rows(z2[q]);
+    } else if ((q -= MLP_HID) < MLP_HID) {
+      out[MLP_PARAMS - 1 - MLP_HID + q] = dot_rows(h2[q], sdy);
+    } else if (q == MLP_HID) {
+      out[MLP_PARAMS - 1] = sum_rows(sdy);
+    } else {
+      out[MLP_PARAMS] = sum_rows(ssq);
+    }
   }
 }
 
-// Sum the block partials in order; Adam update when lr > 0 (step from 1).
-__global__ __launch_bounds__(256) void k_mlp_adam(const float* __restrict__ partial, int nblk,
-                                                  float* __restrict__ P, float* __restrict__ m,
-                                                  float* __restrict__ v, float* __restrict__ grad_out, float lr,
-                                                  int step, float* __restrict__ loss_out, int B) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p > MLP_PARAMS) return;
+// Sums of the blocks' partials, 64 parameters per workgroup and 16 interleaved
+// runs of blocks per parameter, added in a fixed order; Adam update when
+// lr > 0 (c1, c2: 1 - beta^step).
+constexpr int ADAM_RUNS = 16;
+__global__ __launch_bounds__(64 * ADAM_RUNS) void k_mlp_adam(const float* __restrict__ partial, int nblk,
+                                                             float* __restrict__ P, float* __restrict__ m,
+                                                             float* __restrict__ v, float* __restrict__ grad_out,
+                                                             float lr, float c1, float c2,
+                                                             float* __restrict__ loss_out, int B) {
+  __shared__ float part[ADAM_RUNS][64];
+  const int lane = threadIdx.x & 63, run = threadIdx.x >> 6;
+  const int p = blockIdx.x * 64 + lane;
+  float s = 0.f;
+  if (p <= MLP_PARAMS) {
+#pragma unroll 8
+    for (int k = run; k < nblk; k += ADAM_RUNS) s += partial[(size_t)k * (MLP_PARAMS + 1) + p];
+  }
+  part[run][lane] = s;
+  __syncthreads();
+  if (run != 0 || p > MLP_PARAMS) return;
   float g = 0.f;
-  for (int k = 0; k < nblk; ++k) g += partial[(size_t)k * (MLP_PARAMS + 1) + p];
+#pragma unroll
+  for (int k = 0; k < ADAM_RUNS; ++k) g += part[k][lane];
   if (p == MLP_PARAMS) {
     if (loss_out) *loss_out = g / (float)B;
     return;
@@ -162,21 +230,10 @@ __global__ __launch_bounds__(256) void k_mlp_adam(const float* __restrict__ part
     const float vv = b2 * v[p] + (1.f - b2) * g * g;
     m[p] = mm;
     v[p] = vv;
-    const float mh = mm / (1.f - powf(b1, (float)step));
-    const float vh = vv / (1.f - powf(b2, (float)step));
+    const float mh = mm / c1;
+    const float vh = vv / c2;
     P[p] -= lr * mh / (sqrtf(vh) + eps);
   }
-}
-
-// Mini-batch indices: splitmix64 of (seed, step, b) mod n.
-__global__ void k_batch_indices(uint32_t* __restrict__ idx, int B, uint32_t n, uint64_t seed, int step) {
-  const int b = blockIdx.x * 256 + threadIdx.x;
-  if (b >= B) return;
-  uint64_t z = seed + ((uint64_t)step * (uint64_t)B + (uint64_t)b + 1ull) * 0x9E3779B97F4A7C15ull;
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-  z ^= z >> 31;
-  idx[b] = (uint32_t)(z % n);
 }
 
 __global__ void k_standardise(const float* __restrict__ raw, float* __restrict__ x, uint32_t n,
@@ -394,35 +451,20 @@ struct DevBuf {
   }
 };
 
-// One forward/backward over `B` samples (idx or the first B rows) and either
-// an Adam step (lr > 0) or only the gradient; loss to *loss.
-int train_pass(const float* x, const float* t, const uint32_t* idx, int B, float* P, float* mo, float* ve,
-               float* grad, float lr, int step, float* loss_dev, const TrainBufs& tb, float* partial) {
-  k_mlp_fwd_bwd<<<(B + 255) / 256, 256>>>(P, x, t, idx, B, tb);
-  PSL_LAUNCH_CHECK();
+// One forward/backward over `B` rows and either an Adam step (lr > 0) or only
+// the gradient; loss to *loss.
+int train_pass(const float* x, const float* t, const BatchDraw& draw, int B, float* P, float* mo, float* ve,
+               float* grad, float lr, int step, float* loss_dev, float* partial) {
   const int nblk = (B + CHUNK - 1) / CHUNK;
-  k_mlp_grad_partial<<<nblk, 256>>>(x, idx, B, tb, partial);
+  k_mlp_batch<<<nblk, 256>>>(P, x, t, draw, B, partial);
   PSL_LAUNCH_CHECK();
-  k_mlp_adam<<<(MLP_PARAMS + 1 + 255) / 256, 256>>>(partial, nblk, P, mo, ve, grad, lr, step, loss_dev, B);
+  const float c1 = (float)(1.0 - std::pow((double)0.9f, step)), c2 = (float)(1.0 - std::pow((double)0.999f, step));
+  k_mlp_adam<<<(MLP_PARAMS + 1 + 63) / 64, 64 * ADAM_RUNS>>>(partial, nblk, P, mo, ve, grad, lr, c1, c2, loss_dev, B);
   PSL_LAUNCH_CHECK();
   return PSL_OK;
 }
 
-int alloc_train(int B, DevBuf (&bufs)[7], TrainBufs& tb, float*& partial) {
-  const size_t h = (size_t)B * MLP_HID * sizeof(float);
-  int rc = bufs[0].alloc(h);
-  if (!rc) rc = bufs[1].alloc(h);
-  if (!rc) rc = bufs[2].alloc(h);
-  if (!rc) rc = bufs[3].alloc(h);
-  if (!rc) rc = bufs[4].alloc((size_t)B * sizeof(float));
-  if (!rc) rc = bufs[5].alloc((size_t)B * sizeof(float));
-  if (!rc) rc = bufs[6].alloc((size_t)((B + CHUNK - 1) / CHUNK) * (MLP_PARAMS + 1) * sizeof(float));
-  if (rc) return rc;
-  tb = {bufs[0].as<float>(), bufs[1].as<float>(), bufs[2].as<float>(), bufs[3].as<float>(), bufs[4].as<float>(),
-        bufs[5].as<float>()};
-  partial = bufs[6].as<float>();
-  return PSL_OK;
-}
+size_t partial_bytes(int B) { return (size_t)((B + CHUNK - 1) / CHUNK) * (MLP_PARAMS + 1) * sizeof(float); }
 
 }  // namespace
 
@@ -480,17 +522,15 @@ int psl_mlp_get_params(const psl_mlp* m, float* params, float* mean, float* std_
 
 int psl_mlp_loss_grad(const psl_mlp* m, const float* x_dev, const float* t_dev, int n, double* loss, float* grad) {
   PSL_CHECK_ARG(m && x_dev && t_dev && n > 0, "bad arguments");
-  DevBuf bufs[7], dP, dG, dL;
-  TrainBufs tb;
-  float* partial = nullptr;
-  int rc = alloc_train(n, bufs, tb, partial);
+  DevBuf dpart, dP, dG, dL;
+  int rc = dpart.alloc(partial_bytes(n));
   if (!rc) rc = dP.alloc(sizeof(m->params));
   if (!rc) rc = dG.alloc(sizeof(m->params));
   if (!rc) rc = dL.alloc(sizeof(float));
   if (rc) return rc;
   PSL_HIP_TRY(hipMemcpy(dP.p, m->params, sizeof(m->params), hipMemcpyHostToDevice));
-  rc = train_pass(x_dev, t_dev, nullptr, n, dP.as<float>(), nullptr, nullptr, dG.as<float>(), 0.f, 1, dL.as<float>(),
-                  tb, partial);
+  rc = train_pass(x_dev, t_dev, BatchDraw{}, n, dP.as<float>(), nullptr, nullptr, dG.as<float>(), 0.f, 1,
+                  dL.as<float>(), dpart.as<float>());
   if (rc) return rc;
   float l = 0.f;
   PSL_HIP_TRY(hipMemcpy(&l, dL.p, sizeof(float), hipMemcpyDeviceToHost));
@@ -504,10 +544,10 @@ int psl_mlp_train(psl_mlp* m, const float* raw_dev, const float* t_dev, int n, i
   PSL_CHECK_ARG(m && raw_dev && t_dev && n > 0 && batch > 0 && iters > 0 && lr > 0.f, "bad arguments");
   // standardisation from the data (FP64 moments)
   const int nblk_m = 256;
-  DevBuf dpart, dx, didx, dP, dm, dv, dloss, dmean, dinv;
+  DevBuf dpart, dx, dsum, dP, dm, dv, dloss, dmean, dinv;
   int rc = dpart.alloc((size_t)nblk_m * 2 * MLP_IN * sizeof(double));
   if (!rc) rc = dx.alloc((size_t)n * MLP_IN * sizeof(float));
-  if (!rc) rc = didx.alloc((size_t)batch * sizeof(uint32_t));
+  if (!rc) rc = dsum.alloc(partial_bytes(batch));
   if (!rc) rc = dP.alloc(sizeof(m->params));
   if (!rc) rc = dm.alloc(sizeof(m->params));
   if (!rc) rc = dv.alloc(sizeof(m->params));
@@ -536,19 +576,13 @@ int psl_mlp_train(psl_mlp* m, const float* raw_dev, const float* t_dev, int n, i
   k_standardise<<<(uint32_t)(((uint64_t)n * MLP_IN + 255) / 256), 256>>>(raw_dev, dx.as<float>(), (uint32_t)n,
                                                                         dmean.as<float>(), dinv.as<float>());
   PSL_LAUNCH_CHECK();
-  DevBuf bufs[7];
-  TrainBufs tb;
-  float* partial = nullptr;
-  rc = alloc_train(batch, bufs, tb, partial);
-  if (rc) return rc;
   PSL_HIP_TRY(hipMemcpy(dP.p, m->params, sizeof(m->params), hipMemcpyHostToDevice));
   PSL_HIP_TRY(hipMemset(dm.p, 0, sizeof(m->params)));
   PSL_HIP_TRY(hipMemset(dv.p, 0, sizeof(m->params)));
   for (int it = 0; it < iters; ++it) {
-    k_batch_indices<<<(batch + 255) / 256, 256>>>(didx.as<uint32_t>(), batch, (uint32_t)n, seed, it);
-    PSL_LAUNCH_CHECK();
-    rc = train_pass(dx.as<float>(), t_dev, didx.as<uint32_t>(), batch, dP.as<float>(), dm.as<float>(),
-                    dv.as<float>(), nullptr, lr, it + 1, dloss.as<float>() + it, tb, partial);
+    rc = train_pass(dx.as<float>(), t_dev, BatchDraw{true, (uint32_t)n, ~0ull / (uint64_t)n, seed, it}, batch,
+                    dP.as<float>(), dm.as<float>(), dv.as<float>(), nullptr, lr, it + 1, dloss.as<float>() + it,
+                    dsum.as<float>());
     if (rc) return rc;
   }
   PSL_HIP_TRY(hipMemcpy(m->params, dP.p, sizeof(m->params), hipMemcpyDeviceToHost));

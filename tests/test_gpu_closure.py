@@ -58,6 +58,40 @@ def test_training_gradient_matches_oracle(psl):
     assert err < 1e-4
 
 
+@pytest.mark.parametrize("rows", [1, 63, 64, 65, 129, 1023, 1025, 16384])
+def test_training_gradient_at_workgroup_edges(psl, rows):
+    """Batches around the 64 rows of a workgroup and the 16 runs of workgroups
+    that the update adds: FP32 sums of up to 16384 terms of either sign, each
+    rounded within 6e-8 of the partial sums, stay within 1e-5 of the largest
+    component of the FP64 gradient."""
+    P = psl
+    rng = np.random.default_rng(rows)
+    p = (C.init_params(3) + rng.normal(0, 0.05, C.N_PARAM)).astype(np.float32)
+    x = rng.normal(0, 1, (rows, C.N_IN)).astype(np.float32)
+    t = rng.normal(0.5, 1, rows).astype(np.float32)
+    loss, g = P.MLP(p).loss_grad(x, t)
+    p64, x64, t64 = p.astype(np.float64), x.astype(np.float64), t.astype(np.float64)
+    g_ref = C.mlp_grad(p64, x64, t64)
+    assert abs(loss / C.mlp_loss(p64, x64, t64) - 1) < 1e-5
+    assert np.max(np.abs(g - g_ref)) < 1e-5 * np.max(np.abs(g_ref))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 1000003])
+def test_training_draws_rows_modulo_any_count(psl, n):
+    """The batch rows (a 64-bit remainder from a reciprocal): with a target that
+    is the row number and a network of constant zero output, the first loss is
+    the mean square of the drawn row numbers."""
+    P = psl
+    raw = np.random.default_rng(1).normal(0, 1, (n, C.N_IN)).astype(np.float32)
+    t = (np.arange(n) % 4096).astype(np.float32)
+    net = P.MLP(np.zeros(C.N_PARAM, np.float32))
+    hist = net.train(P.DeviceBuffer.from_array(raw), P.DeviceBuffer.from_array(t), n, batch=700, iters=1, lr=1e-3,
+                     seed=(1 << 63) + 12345)
+    rows = _splitmix_indices((1 << 63) + 12345, 0, 700, n)
+    want = np.mean(t[rows].astype(np.float64) ** 2)
+    assert abs(hist[0] - want) <= 1e-5 * want
+
+
 def test_adam_training_matches_oracle(psl):
     P = psl
     rng = np.random.default_rng(12)
