@@ -11,6 +11,7 @@
 //
 // Layout: fArray(q, cell) at f[q * n + cell]; ijk[3][n]; nbr[7][n].
 #include "psl_internal.h"
+#include "psl_stream.h"
 
 #include <algorithm>
 #include <atomic>
@@ -164,10 +165,21 @@ __global__ void k_eso_adjacency(const int* __restrict__ nbr, uint32_t n, uint8_t
   adj[c] = m;
 }
 
-template <class St, bool FLIP>
+// Bound by the traffic of the 27 populations' rows: 4.45 TB/s of them in FP16 on
+// a dense 256^3 box (41 GLUPS), 3.4 on the sparse levels, whose rows of tens of
+// cells split a wave's stores over many lines.  Two choices follow from the
+// latter: blocks are dealt to the XCDs four at a time, so that the lines at
+// their borders are shared in one L2 (6-level sphere, FP16: 60.6 ms per coarse
+// step one at a time, 59.8 / 60.0 / 60.4 at 4 / 16 / 64, one range per XCD 64),
+// and each access is a scalar row base and a 32-bit offset, the populations
+// staying storage words until the moments, which takes 89 VGPRs instead of 114
+// (61.4 -> 60.6 ms).  Held to 80 or 72 VGPRs it spills (71 and 97 ms).  WIDE:
+// rows of 4 GiB and more.
+template <class St, bool FLIP, bool WIDE>
 __global__ __launch_bounds__(256) void k_eso_update(typename St::T* __restrict__ f, EsoParams p) {
   typedef typename St::T T;
-  const uint32_t cell = blockIdx.x * 256u + threadIdx.x;
+  typedef typename std::conditional<WIDE, size_t, uint32_t>::type Off;
+  const uint32_t cell = xcd_block_chunked<4>(blockIdx.x, gridDim.x) * 256u + threadIdx.x;
   if (cell >= p.n) return;
   const int fl = p.flags ? p.flags[cell] : 0;
   int kind = fl & 7;
@@ -175,16 +187,16 @@ __global__ __launch_bounds__(256) void k_eso_update(typename St::T* __restrict__
   if (kind == KIND_GHOST || kind == KIND_COVERED) kind = KIND_GIVEN_NONE;
   uint32_t slot[8];
   eso_slots_adj(p, cell, slot);
-  float v[27];
+  auto at = [&](int row, int s) { return (T*)((char*)(f + (size_t)row * p.n) + (Off)slot[s] * (Off)sizeof(T)); };
+  Word<St> r[27];
 #pragma unroll
-  for (int q = 0; q < 27; ++q) {
-    const int fi = FLIP ? q : opp(q);
-    v[q] = St::load(f[(size_t)fi * p.n + slot[ESO_READ[q]]]);
-  }
+  for (int q = 0; q < 27; ++q) r[q] = (Word<St>)ld<T, false>(at(FLIP ? q : opp(q), ESO_READ[q]));
   Relax rx{p.omega, p.tau, p.cs};
+  float v[27];
   if (kind == KIND_FLUID) {
-    collide<St::W_OFF>(v, rx, p.cs);
+    collide_with_moments<St::W_OFF>(v, raw_moments_words<St>(r), rx, p.cs);
   } else {
+    words_to_float<St>(r, v);
     if (St::W_OFF) {
 #pragma unroll
       for (int q = 0; q < 27; ++q) v[q] += weight(q);
@@ -200,10 +212,7 @@ __global__ __launch_bounds__(256) void k_eso_update(typename St::T* __restrict__
     }
   }
 #pragma unroll
-  for (int q = 0; q < 27; ++q) {
-    const int fi = FLIP ? opp(q) : q;
-    f[(size_t)fi * p.n + slot[ESO_WRITE[q]]] = St::store(v[q]);
-  }
+  for (int q = 0; q < 27; ++q) st<T, false>(at(FLIP ? opp(q) : q, ESO_WRITE[q]), St::store(v[q]));
   if (p.rec) {
     const int r = rec_index(p.rec_mask, p.rec_base, cell);
     if (r >= 0) rec_store<St>(p.rec, (uint32_t)r, v);
@@ -1013,8 +1022,14 @@ template <class St>
 static int eso_update(psl_diad* d, bool child_records) {
   const EsoParams p = eso_params(d, child_records);
   const uint32_t nb = (uint32_t)((d->n + 255) / 256);
-  if (d->flipper) k_eso_update<St, true><<<nb, 256, 0, d->stream>>>((typename St::T*)d->f, p);
-  else k_eso_update<St, false><<<nb, 256, 0, d->stream>>>((typename St::T*)d->f, p);
+  typename St::T* f = (typename St::T*)d->f;
+  if ((uint64_t)p.n * sizeof(typename St::T) > 0xffffffffull) {
+    if (d->flipper) k_eso_update<St, true, true><<<nb, 256, 0, d->stream>>>(f, p);
+    else k_eso_update<St, false, true><<<nb, 256, 0, d->stream>>>(f, p);
+  } else {
+    if (d->flipper) k_eso_update<St, true, false><<<nb, 256, 0, d->stream>>>(f, p);
+    else k_eso_update<St, false, false><<<nb, 256, 0, d->stream>>>(f, p);
+  }
   PSL_LAUNCH_CHECK();
   // the records this update wrote hold its values; the others are behind
   d->child.fresh = p.rec != nullptr;
