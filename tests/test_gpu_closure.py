@@ -138,6 +138,25 @@ def test_matrix_core_inference_matches_oracle(psl):
     assert err <= 0.03 * np.max(np.abs(y_ref)) + 0.02
 
 
+@pytest.mark.parametrize("n,r", [(12, 1), (12, 3), (60, 20), (258, 2), (258, 129), (257, 257)])
+def test_les_filter_at_workgroup_edges(psl, n, r):
+    """Runs of coarse cells that fill a workgroup's 256 lanes, leave a remainder
+    (129 cells in runs of 128), one cell per run, and a width beyond the lanes.
+    Means of FP64 sums rounded to FP32 stay within 1e-6; the stresses are
+    differences of such means, absolute within 1e-7 of the 1e-2 they come from."""
+    P = psl
+    rng = np.random.default_rng(n + r)
+    fx, fy = n + 2, n + 1
+    shape = (n, fy, fx)
+    f = [rng.uniform(0.97, 1.03, shape), *(rng.uniform(-0.1, 0.1, shape) for _ in range(3))]
+    f = [a.astype(np.float32) for a in f]
+    m = n // r
+    got = P.les_filter(*[P.DeviceBuffer.from_array(a.ravel()) for a in f], fx, fy, n, r).download((10, m, m, m))
+    rb, a, b, c, tau = C.les_filter(*[x.astype(np.float64)[:, :n, :n] for x in f], r)
+    ref = np.concatenate([np.stack([rb, a, b, c]), tau])
+    assert np.max(np.abs(got - ref) - 1e-6 * np.abs(ref)) < 1e-9
+
+
 def test_les_filter_and_targets_match_oracle(psl):
     P = psl
     rng = np.random.default_rng(14)
