@@ -262,7 +262,7 @@ int psl_grid_check_health(psl_grid* grid, int64_t* bad_cells, double* rho_min, d
  * reference steps one grid at a time).  Each grid keeps its own flags, given
  * values, Cs (uniform or per cell) and storage (all grids share the storage);
  * one step of all grids is one bulk launch over the blocks of every grid and
- * one launch over all boundary lists (or one fused launch).  Steps are captured
+ * (FP16) one launch over all boundary lists, or one fused launch.  Steps are captured
  * in hipGraphs of one step and of steps_per_graph steps (default 1000) and
  * replayed, so nsteps steps take nsteps / steps_per_graph + nsteps %
  * steps_per_graph graph launches; a batch whose distributions exceed 192 MB

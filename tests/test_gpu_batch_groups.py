@@ -8,16 +8,17 @@ from periodicshiftlbm_amd import cases
 
 pytestmark = pytest.mark.gpu
 
-# FP16: 270 MB (a group of its own), 27 MB, 95 MB, 101 MB and 1 MB
+# 16-bit: 270 MB (a group of its own), 27 MB, 95 MB, 101 MB and 1 MB
 EDGES = (136, 63, 96, 98, 21)
 
 
-@pytest.mark.parametrize("tuning,order,steps", [(4, 0, 2), (4, 1, 5), (12, 0, 3)])
-def test_grouped_batch_equals_single_grid_steps(psl, tuning, order, steps):
+# box-face cells from the lists (FP16), in the bulk launch (BF16), fused
+@pytest.mark.parametrize("storage,tuning,order,steps", [("f16", 4, 0, 2), ("bf16", 4, 1, 5), ("f16", 12, 0, 3)])
+def test_grouped_batch_equals_single_grid_steps(psl, storage, tuning, order, steps):
     P = psl
     doms = [{"shape": (2 * L, L, L), "nu": 1e-3 * (1 + i), "u_inlet": 0.04, "diameter": 0.25 * L,
              "center": (0.5 * L,) * 3} for i, L in enumerate(EDGES)]
-    batched = [cases.domain_grid(d, "f16")[0] for d in doms]
+    batched = [cases.domain_grid(d, storage)[0] for d in doms]
     assert sum(54 * g.n for g in batched) > 2 * 192 << 20
     b = P.Batch(batched)
     b.set_tuning(tuning, order)
@@ -25,7 +26,7 @@ def test_grouped_batch_equals_single_grid_steps(psl, tuning, order, steps):
     b.step(1)
     b.step(steps + 1)
     for d, g in zip(doms, batched):
-        alone = cases.domain_grid(d, "f16")[0]
+        alone = cases.domain_grid(d, storage)[0]
         P.updateGrid([alone], 2 * steps + 2)
         assert g.shifter.tolist() == alone.shifter.tolist()
         nbad = int(np.count_nonzero(g.get_f().view(np.uint32) != alone.get_f().view(np.uint32)))
