@@ -103,11 +103,11 @@ def in_step_kernel_ms(P, g, steps: int) -> float:
 
 def batch_leg(P, cases, steps: int, autotune_steps: int, storage: str = "f16", avg_steps: int = 2500,
               avg_every: int = 100):
-    """64 sphere-in-channel domains of uneven size advanced by replays of a
-    hipGraph of 1000 captured steps; aggregate MLUPS, its HBM fraction, and
+    """64 sphere-in-channel domains of uneven size advanced as one batch (2.5 GB
+    in FP16: in groups that fit the last-level cache); aggregate MLUPS, its HBM fraction, and
     per-domain drag coefficient averaged over avg_steps steps after the timed
     run.  The autotuner searches kernel variant, grid order, cells per thread
-    and tile order; the multi-step graph is captured in an untimed warm-up."""
+    and tile order."""
     doms = cases.batch_domains()
     grids = [cases.domain_grid(d, storage)[0] for d in doms]
     b = P.Batch(grids)
@@ -119,7 +119,7 @@ def batch_leg(P, cases, steps: int, autotune_steps: int, storage: str = "f16", a
                                 for ti in range(2) for c in range(2) for od in range(2)}}
     cells, blocks, nbnd = b.census()
     if steps >= b.steps_per_graph:
-        b.step(b.steps_per_graph)  # captures the multi-step graph
+        b.step(b.steps_per_graph)  # untimed warm-up (captures the multi-step graph of a batch that uses one)
     for g in grids:  # restart from rest after tuning and warm-up
         P.fill_equilibrium(g)
     P.synchronize()
@@ -145,7 +145,7 @@ def batch_leg(P, cases, steps: int, autotune_steps: int, storage: str = "f16", a
             "cells": cells, "boundary_cells": nbnd, "steps": steps, "storage": storage, "autotune": tune,
             "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": achieved / HBM_PEAK_GBS, "bytes_per_cell": BYTES_PER_UPDATE[storage],
-                         "note": "whole step (all kernels of the replayed graph) over all domains"},
+                         "note": "whole step (all kernels) over all domains"},
             "working_set_bytes": cells * 27 * (4 if storage == "f32" else 2),
             "drag_coefficient_mean": [round(float(c), 5) for c in cd],
             "drag_average": {"after_step": steps, "steps": avg_steps, "every": avg_every},
@@ -602,7 +602,8 @@ def main():
         lo, hi = cases.sphere_box()
         fx = g.momentum_exchange(lo, hi)[0]
         # the dominant launch (k_ps_fused updates the bulk and the boundary
-        # list, k_ps_bulk the bulk only) inside as many steps again, an event
+        # list, k_ps_bulk the bulk, and the list where it updates it in place,
+        # which is left out of its bytes) inside as many steps again, an event
         # pair around each launch; beside it, 256 launches back to back with
         # the shifter advancing (faster: no other kernels between them)
         avg_ms = in_step_kernel_ms(P, g, args.steps)

@@ -192,8 +192,10 @@ int psl_device_free(void* ptr);
 int psl_device_upload(void* dst_device, const void* src_host, size_t bytes);
 int psl_device_download(void* dst_host, const void* src_device, size_t bytes);
 /* Local-update variants (bits): non-temporal loads / stores and XCD-contiguous
- * block order in the bulk kernel; FUSED_BOUNDARY updates the box-face list in
- * the same launch as the bulk instead of a second launch. */
+ * block order in the bulk kernel; FUSED_BOUNDARY updates the box-face list by
+ * workgroups of its own between the bulk's.  Without it the bulk kernel updates
+ * those cells in place or stages them for a second launch, by storage and size;
+ * the non-temporal bits apply where it stages them or there are none. */
 enum {
   PSL_TUNE_NT_LOAD = 1,
   PSL_TUNE_NT_STORE = 2,

@@ -542,8 +542,9 @@ class GridStruct:
 
 
 class Batch:
-    """Many GridStructs advanced together by replays of captured hipGraphs
-    (one of a single step, one of steps_per_graph steps)."""
+    """Many GridStructs advanced together: by replays of captured hipGraphs (one
+    of a single step, one of steps_per_graph steps), or, beyond the last-level
+    cache, in groups of grids that fit it."""
 
     def __init__(self, grids: Sequence[GridStruct]):
         self.grids = list(grids)  # keep the grids alive
