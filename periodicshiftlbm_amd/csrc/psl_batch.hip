@@ -31,6 +31,7 @@
 // first) and the kernel variant are chosen by psl_batch_autotune, and with
 // them the cells per thread and the tile order by psl_batch_autotune_layouts.
 #include "psl_internal.h"
+#include "psl_batch_run.h"
 #include "psl_stream.h"
 
 #include <algorithm>
@@ -198,6 +199,7 @@ struct psl_batch {
   BatchEntry* d_order = nullptr;
   uint32_t total_blocks = 0, total_bblocks = 0, total_bnd = 0, total_fused = 0;
   int64_t total_cells = 0;
+  std::vector<uint32_t> launch_order;  // grids in the order of the launch tables
   BatchGroup whole;                // all grids
   std::vector<BatchGroup> groups;  // at least one
   hipGraph_t graph = nullptr;  // one step
@@ -310,14 +312,12 @@ int enqueue_step(psl_batch* b, const BatchGroup& G, int s, int steps) {
   return PSL_OK;
 }
 
-int enqueue_run(psl_batch* b, const BatchGroup& G, int steps) {
-  int rc = PSL_OK;
-  for (int s = 0; s < steps && rc == PSL_OK; ++s) switch (b->storage) {
-      case PSL_F32: rc = enqueue_step<StF32>(b, G, s, steps); break;
-      case PSL_F16DEV: rc = enqueue_step<StF16>(b, G, s, steps); break;
-      default: rc = enqueue_step<StBF16>(b, G, s, steps); break;
-    }
-  return rc;
+int enqueue_dispatch(psl_batch* b, const BatchGroup& G, int s, int steps) {
+  switch (b->storage) {
+    case PSL_F32: return enqueue_step<StF32>(b, G, s, steps);
+    case PSL_F16DEV: return enqueue_step<StF16>(b, G, s, steps);
+    default: return enqueue_step<StBF16>(b, G, s, steps);
+  }
 }
 
 template <class T>
@@ -337,7 +337,7 @@ int capture_steps(psl_batch* b, int steps, hipGraph_t* graph_out, hipGraphExec_t
   b->stream = cap;
   hipError_t e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
   int rc = PSL_OK;
-  if (e == hipSuccess) rc = enqueue_run(b, b->whole, steps);
+  for (int s = 0; e == hipSuccess && rc == PSL_OK && s < steps; ++s) rc = enqueue_dispatch(b, b->whole, s, steps);
   hipGraph_t graph = nullptr;
   hipError_t e2 = hipStreamEndCapture(cap, &graph);
   b->stream = saved;
@@ -412,7 +412,7 @@ int build_batch(psl_batch* b) {
   }
   // groups of consecutive grids of the launch order whose distributions fit
   // GROUP_BYTES together (a larger grid is a group of its own), of about equal size
-  std::vector<uint32_t> dom(order.begin(), order.end());
+  b->launch_order.assign(order.begin(), order.end());
   const size_t cell_bytes = 27 * storage_bytes(b->storage);
   auto bytes_of = [&](int d) { return (size_t)b->grids[d]->info.cellCount * cell_bytes; };
   size_t total_bytes = 0;
@@ -503,7 +503,7 @@ int build_batch(psl_batch* b) {
   if (!rc) rc = upload(&b->d_faces, faces);
   if (!rc) rc = upload(&b->d_fbase, fbase);
   if (!rc) rc = upload(&b->d_delta, delta);
-  if (!rc) rc = upload(&b->d_dom, dom);
+  if (!rc) rc = upload(&b->d_dom, b->launch_order);
   if (!rc) rc = upload(&b->d_block_domain, block_domain);
   if (!rc) rc = upload(&b->d_block_tile, block_tile);
   if (!rc) rc = upload(&b->d_bblock_domain, bblock_domain);
@@ -548,6 +548,12 @@ int upload_shifts(psl_batch* b) {
   PSL_HIP_TRY(hipMemcpyAsync(b->d_shift, sh.data(), sh.size() * sizeof(int), hipMemcpyHostToDevice, b->stream));
   PSL_HIP_TRY(hipStreamSynchronize(b->stream));
   return PSL_OK;
+}
+
+// The host shifters of one group's grids, `steps` steps on.
+void advance_shifters(psl_batch* b, const BatchGroup& G, int steps) {
+  for (uint32_t at = G.dom0; at < G.dom0 + G.ndom; ++at)
+    for (int s = 0; s < steps; ++s) (void)psl_apply_streaming(b->grids[b->launch_order[at]]);
 }
 
 }  // namespace
@@ -611,28 +617,23 @@ int psl_batch_step(psl_batch* b, int nsteps) {
   // a batch beyond the cache: every group of grids runs all its steps in turn,
   // launched as they are (a group's launches are long enough to hide their own
   // enqueueing); one step of everything gains nothing from groups
-  if (nsteps > 1 && b->groups.size() > 1) {
-    for (const BatchGroup& G : b->groups) {
-      rc = enqueue_run(b, G, nsteps);
-      if (rc) return rc;
-    }
-    for (psl_grid* g : b->grids)
-      for (int s = 0; s < nsteps; ++s) psl_apply_streaming(g);
-    return PSL_OK;
-  }
+  if (nsteps > 1 && b->groups.size() > 1)
+    return run_groups(
+        b->groups.size(), nsteps, [&](size_t g, int s) { return enqueue_dispatch(b, b->groups[g], s, nsteps); },
+        [&](size_t g, int n) { advance_shifters(b, b->groups[g], n); });
   // whole graphs of steps_per_graph steps, then single steps
   const int k = b->steps_per_graph;
   if (k > 1 && nsteps >= k && !b->exec_k) {
     rc = capture_steps(b, k, &b->graph_k, &b->exec_k);
     if (rc) return rc;
   }
-  int left = nsteps;
-  if (k > 1)
-    for (; left >= k; left -= k) PSL_HIP_TRY(hipGraphLaunch(b->exec_k, b->stream));
-  for (; left > 0; --left) PSL_HIP_TRY(hipGraphLaunch(b->exec, b->stream));
-  for (psl_grid* g : b->grids)
-    for (int s = 0; s < nsteps; ++s) psl_apply_streaming(g);
-  return PSL_OK;
+  return run_graphs(
+      nsteps, k,
+      [&](int n) -> int {
+        PSL_HIP_TRY(hipGraphLaunch(n > 1 ? b->exec_k : b->exec, b->stream));
+        return PSL_OK;
+      },
+      [&](int n) { advance_shifters(b, b->whole, n); });
 }
 
 int psl_batch_set_tuning(psl_batch* b, int tuning, int order) {
