@@ -410,27 +410,10 @@ int build_batch(psl_batch* b) {
     ntile[d] = (uint32_t)((b->grids[d]->info.cellCount + tile_cells - 1) / tile_cells);
     max_tiles = std::max(max_tiles, ntile[d]);
   }
-  // groups of consecutive grids of the launch order whose distributions fit
-  // GROUP_BYTES together (a larger grid is a group of its own), of about equal size
   b->launch_order.assign(order.begin(), order.end());
-  const size_t cell_bytes = 27 * storage_bytes(b->storage);
-  auto bytes_of = [&](int d) { return (size_t)b->grids[d]->info.cellCount * cell_bytes; };
-  size_t total_bytes = 0;
-  for (int d : order) total_bytes += bytes_of(d);
-  const size_t want = (total_bytes + GROUP_BYTES - 1) / GROUP_BYTES;
-  const size_t share = (total_bytes + want - 1) / want;
-  std::vector<size_t> ends;  // launch-order positions past each group
-  size_t in_group = 0, before = 0;
-  for (int at = 0; at < nd; ++at) {
-    const size_t bytes = bytes_of(order[at]);
-    if (in_group && (in_group + bytes > GROUP_BYTES || before + bytes / 2 > share * (ends.size() + 1))) {
-      ends.push_back((size_t)at);
-      in_group = 0;
-    }
-    in_group += bytes;
-    before += bytes;
-  }
-  ends.push_back((size_t)nd);
+  std::vector<size_t> bytes;
+  for (int d : order) bytes.push_back((size_t)b->grids[d]->info.cellCount * 27 * storage_bytes(b->storage));
+  const std::vector<size_t> ends = group_ends(bytes, GROUP_BYTES);
   std::vector<BatchEntry> fused;
   size_t at0 = 0;
   b->groups.clear();

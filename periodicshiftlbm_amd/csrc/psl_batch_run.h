@@ -1,10 +1,42 @@
-// Order of the launches of a batch call and what it leaves in the host
-// shifters (plain C++, no HIP types).
+// The groups of grids of a batch, the order of a call's launches and what it
+// leaves in the host shifters (plain C++, no HIP types).
 #pragma once
 
 #include <cstddef>
+#include <vector>
 
 namespace psl {
+
+// Groups of consecutive grids that are stepped together, as the positions past
+// each: grids of `bytes` in turn, as many as fit `limit` together, the groups
+// of a run of them about equal in size.  A grid above `limit` is a group of its
+// own and ends the run, so that its size does not count in the shares of the
+// others.
+inline std::vector<size_t> group_ends(const std::vector<size_t>& bytes, size_t limit) {
+  std::vector<size_t> ends;
+  for (size_t at = 0; at < bytes.size();) {
+    if (bytes[at] > limit) {
+      ends.push_back(++at);
+      continue;
+    }
+    size_t end = at, total = 0;
+    for (; end < bytes.size() && bytes[end] <= limit; ++end) total += bytes[end];
+    const size_t want = total > limit ? (total + limit - 1) / limit : 1;
+    const size_t share = (total + want - 1) / want;
+    size_t in_group = 0, before = 0, groups = 1;
+    for (; at < end; ++at) {
+      if (in_group && (in_group + bytes[at] > limit || before + bytes[at] / 2 > share * groups)) {
+        ends.push_back(at);
+        in_group = 0;
+        ++groups;
+      }
+      in_group += bytes[at];
+      before += bytes[at];
+    }
+    ends.push_back(end);
+  }
+  return ends;
+}
 
 // `steps` steps of each of `groups` groups of grids, one group after the
 // other.  enqueue(g, s) launches step s of group g and returns 0 or an error

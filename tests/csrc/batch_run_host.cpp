@@ -1,8 +1,13 @@
-// Host build of the batch call's launch order (psl_batch_run.h) with a launch
-// that fails where it is told to.  Test infrastructure only.
+// Host build of the batch's groups and launch order (psl_batch_run.h), with a
+// launch that fails where it is told to.  Test infrastructure only.
 #include "../../periodicshiftlbm_amd/csrc/psl_batch_run.h"
 
 extern "C" {
+int br_ends(int n, const long long* bytes, long long limit, int* ends) {
+  const std::vector<size_t> e = psl::group_ends(std::vector<size_t>(bytes, bytes + n), (size_t)limit);
+  for (size_t i = 0; i < e.size(); ++i) ends[i] = (int)e[i];
+  return (int)e.size();
+}
 // moved[g]: steps that group g's shifters moved; launched[g]: steps launched.
 int br_groups(int groups, int steps, int fail_group, int fail_step, int* launched, int* moved) {
   return psl::run_groups(

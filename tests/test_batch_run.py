@@ -1,6 +1,8 @@
-"""What a batch call leaves in the host shifters when a launch fails (host build
-of psl_batch_run.h): every group of grids stands at the steps launched for it,
-in the form of groups and in that of graphs."""
+"""The groups and launches of a batch call (host build of psl_batch_run.h): groups
+of grids that fit the limit together, of about equal size, whatever larger grids
+stand between them; and the host shifters when a launch fails: every group of
+grids stands at the steps launched for it, in the form of groups and in that of
+graphs."""
 import ctypes
 import os
 import subprocess
@@ -41,3 +43,33 @@ def test_graph_shifters_follow_the_launched_steps(host, steps, many, fail, want)
     rc = host.br_graphs(steps, many, fail, ctypes.byref(launched), ctypes.byref(moved))
     assert rc == (0 if fail < 0 else 7)
     assert launched.value == moved.value == want
+
+
+def _ends(host, sizes, limit):
+    b, out = np.array(sizes, np.int64), np.zeros(len(sizes), np.int32)
+    n = host.br_ends(len(sizes), b.ctypes.data_as(ctypes.c_void_p), ctypes.c_longlong(limit),
+                     out.ctypes.data_as(ctypes.c_void_p))
+    return out[:n].tolist()
+
+
+def test_groups_beside_a_larger_grid(host):
+    """2 GB ahead of 40 grids of 5 MB: those fill two groups, not one each."""
+    assert _ends(host, [2000] + [5] * 40, 192) == [1, 21, 41]
+    assert _ends(host, [5] * 40 + [2000], 192) == [20, 40, 41]
+
+
+@pytest.mark.parametrize("seed", range(20))
+def test_groups_fill_the_limit(host, seed):
+    """Every grid is in one group; a group of several fits the limit; of two
+    neighbouring groups of smaller grids, one is over a quarter of the limit."""
+    rng = np.random.default_rng(seed)
+    limit = 192
+    sizes = np.where(rng.random(60) < 0.1, rng.integers(193, 3000, 60), rng.integers(1, 60, 60)).tolist()
+    ends = _ends(host, sizes, limit)
+    assert ends[-1] == len(sizes) and all(a < b for a, b in zip(ends, ends[1:]))
+    groups = [sizes[a:b] for a, b in zip([0] + ends, ends)]
+    for g in groups:
+        assert len(g) == 1 or sum(g) <= limit
+    for a, b in zip(groups, groups[1:]):
+        if max(a + b) <= limit:
+            assert max(sum(a), sum(b)) > limit // 4
