@@ -296,7 +296,11 @@ __global__ __launch_bounds__(256) void k_mlp_eval(const MlpNet* __restrict__ net
 // n m^2 lanes share them (a thread per coarse cell read 4 bytes per line and
 // left the chip to 128 workgroups: 259 us for 256^3 filtered 8 times, 270 MB).
 // The columns then add in fine x order, one (cell, quantity) per thread.
-constexpr int FILTER_LANES = 256, FILTER_SUMS = 10;
+// Widths under FILTER_MIN gain nothing from it: a wave of k_les_filter_cells
+// reads most of its lines there too, in one pass without LDS (us per call, cells
+// / lanes: 256^3 by 1 223 / 360, by 2 125 / 141, 258^3 by 3 106 / 145, 256^3 by 4
+// 118 / 77, 300^3 by 5 194 / 163, 256^3 by 8 254 / 61).
+constexpr int FILTER_LANES = 256, FILTER_SUMS = 10, FILTER_MIN = 4;
 __global__ __launch_bounds__(FILTER_LANES) void k_les_filter(const float* __restrict__ rho,
                                                              const float* __restrict__ ux,
                                                              const float* __restrict__ uy,
@@ -354,10 +358,11 @@ __global__ __launch_bounds__(FILTER_LANES) void k_les_filter(const float* __rest
   out[9 * (size_t)mc + o] = (float)(tot[9][t] * inv / R - V * W);
 }
 
-// The filter for widths above FILTER_LANES: a thread per coarse cell.
-__global__ __launch_bounds__(256) void k_les_filter_wide(const float* __restrict__ rho, const float* __restrict__ ux,
-                                                         const float* __restrict__ uy, const float* __restrict__ uz,
-                                                         int fx, int fxy, int r, int m, float* __restrict__ out) {
+// The filter for widths under FILTER_MIN and above FILTER_LANES: a thread per
+// coarse cell.
+__global__ __launch_bounds__(256) void k_les_filter_cells(const float* __restrict__ rho, const float* __restrict__ ux,
+                                                          const float* __restrict__ uy, const float* __restrict__ uz,
+                                                          int fx, int fxy, int r, int m, float* __restrict__ out) {
   const uint32_t c = blockIdx.x * 256u + threadIdx.x;
   const uint32_t mc = (uint32_t)m * m * m;
   if (c >= mc) return;
@@ -669,12 +674,12 @@ int psl_les_filter(const float* rho, const float* ux, const float* uy, const flo
   PSL_CHECK_ARG(r > 0 && n > 0 && n % r == 0 && fine_nx >= n && fine_ny >= n, "bad filter geometry");
   const int m = n / r;
   const uint32_t mc = (uint32_t)m * m * m;
-  if (r <= FILTER_LANES) {
+  if (r >= FILTER_MIN && r <= FILTER_LANES) {
     const int cells = std::min(m, FILTER_LANES / r), runs = (m + cells - 1) / cells;
     k_les_filter<<<(uint32_t)runs * m * m, FILTER_LANES>>>(rho, ux, uy, uz, fine_nx, fine_nx * fine_ny, r, m, cells,
                                                           runs, coarse);
   } else {
-    k_les_filter_wide<<<(mc + 255) / 256, 256>>>(rho, ux, uy, uz, fine_nx, fine_nx * fine_ny, r, m, coarse);
+    k_les_filter_cells<<<(mc + 255) / 256, 256>>>(rho, ux, uy, uz, fine_nx, fine_nx * fine_ny, r, m, coarse);
   }
   PSL_LAUNCH_CHECK();
   PSL_HIP_TRY(hipDeviceSynchronize());

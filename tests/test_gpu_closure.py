@@ -138,10 +138,12 @@ def test_matrix_core_inference_matches_oracle(psl):
     assert err <= 0.03 * np.max(np.abs(y_ref)) + 0.02
 
 
-@pytest.mark.parametrize("n,r", [(12, 1), (12, 3), (60, 20), (258, 2), (258, 129), (257, 257)])
+@pytest.mark.parametrize("n,r", [(12, 1), (12, 3), (12, 4), (60, 20), (258, 2), (260, 4), (260, 5), (258, 129),
+                                 (257, 257)])
 def test_les_filter_at_workgroup_edges(psl, n, r):
     """Runs of coarse cells that fill a workgroup's 256 lanes, leave a remainder
-    (129 cells in runs of 128), one cell per run, and a width beyond the lanes.
+    (65 cells in runs of 64, 52 in runs of 51), one cell per run, and the widths
+    below and beyond the runs, a thread per coarse cell.
     Means of FP64 sums rounded to FP32 stay within 1e-6; the stresses are
     differences of such means, absolute within 1e-7 of the 1e-2 they come from."""
     P = psl
