@@ -43,6 +43,7 @@ struct EsoParams {
   void* srec;                 // source records
   const uint64_t* srec_mask;
   const uint32_t* srec_base;
+  bool deal4;  // the local update's blocks go to the XCDs four at a time
 };
 
 // Interface records: the post-collision storage words of one cell, in q
@@ -168,18 +169,26 @@ __global__ void k_eso_adjacency(const int* __restrict__ nbr, uint32_t n, uint8_t
 // Bound by the traffic of the 27 populations' rows: 4.45 TB/s of them in FP16 on
 // a dense 256^3 box (41 GLUPS), 3.4 on the sparse levels, whose rows of tens of
 // cells split a wave's stores over many lines.  Two choices follow from the
-// latter: blocks are dealt to the XCDs four at a time, so that the lines at
-// their borders are shared in one L2 (6-level sphere, FP16: 60.6 ms per coarse
-// step one at a time, 59.8 / 60.0 / 60.4 at 4 / 16 / 64, one range per XCD 64),
-// and each access is a scalar row base and a 32-bit offset, the populations
-// staying storage words until the moments, which takes 89 VGPRs instead of 114
-// (61.4 -> 60.6 ms).  Held to 80 or 72 VGPRs it spills (71 and 97 ms).  WIDE:
-// rows of 4 GiB and more.
+// latter: on sparse levels blocks are dealt to the XCDs four at a time (p.deal4),
+// so that the lines at their borders are shared in one L2 (6-level sphere, FP16:
+// 60.6 ms per coarse step one at a time, 59.8 / 60.0 / 60.4 at 4 / 16 / 64, one
+// range per XCD 64; levels of 0.1 to 5 M cells gain 0 to 5 %), and each access is
+// a scalar row base and a 32-bit offset, the populations staying storage words
+// until the moments, which takes 89 VGPRs instead of 114 (61.4 -> 60.6 ms).  Held
+// to 80 or 72 VGPRs it spills (71 and 97 ms).  WIDE: rows of 4 GiB and more.
+//
+// A level that fills its box keeps one block at a time: its planes and rows come
+// at regular distances, and at sizes of a power of two the four-block order puts
+// a cell and its +k neighbour on different XCDs, or several streams on one
+// channel (us per update, one / four at a time: FP16 64^3 8.3 / 10.5, 128^3 43.5
+// / 52.2, 256x128x64 42.0 / 48.9; FP32 64^3 8.7 / 10.3, 192x128x128 140 / 149;
+// other sizes gain up to 9 %, FP16 80^3 14.9 / 14.0, 256^3 404 / 394).
 template <class St, bool FLIP, bool WIDE>
 __global__ __launch_bounds__(256) void k_eso_update(typename St::T* __restrict__ f, EsoParams p) {
   typedef typename St::T T;
   typedef typename std::conditional<WIDE, size_t, uint32_t>::type Off;
-  const uint32_t cell = xcd_block_chunked<4>(blockIdx.x, gridDim.x) * 256u + threadIdx.x;
+  const uint32_t block = p.deal4 ? xcd_block_chunked<4>(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint32_t cell = block * 256u + threadIdx.x;
   if (cell >= p.n) return;
   const int fl = p.flags ? p.flags[cell] : 0;
   int kind = fl & 7;
@@ -872,6 +881,7 @@ static EsoParams eso_params(const psl_diad* d, bool child_records = true) {
   p.srec = d->source.n ? d->source.rec : nullptr;
   p.srec_mask = d->source.mask;
   p.srec_base = d->source.base;
+  p.deal4 = (int64_t)d->n != (int64_t)p.nx * p.ny * p.nz;
   return p;
 }
 
