@@ -580,20 +580,29 @@ static void launch_fused(bool les, uint32_t nb, hipStream_t stream, const StepPa
 // runs restore + MBBC (and, for the 16-bit storages, a collision) for that one
 // lane, which costs VALU time; staged, a second launch stores 27 partial lines
 // per cell, which it must fetch again where the grid has left the last-level
-// cache, after a latency of about 10 us.  us per step of the sphere channel,
-// staged against in place: FP32, where the memory leaves the VALU idle,
-// 128x64x64 30.8 / 25.7, 256x128x128 213 / 198, 320x160x160 472 / 388; FP16
-// 128x64x64 27.3 / 24.8, 192x96x96 (91 MB) 49.9 / 51.7, 256x128x128 (216 MB)
-// 91 / 95, 320x160x160 (421 MB) 245 / 227; BF16 26 / 23, 49.8 / 48.4, 92 / 106,
-// 246 / 223, 203x97x121 (123 MB) 62 / 66.  So the 16-bit grids between the
-// latency-bound ones and those beyond the cache are staged.
+// cache, after a latency of about 10 us.  FP32 leaves the VALU idle: in place
+// wins at every size (sphere channel, us per step, staged / in place: 64x32x32
+// 16.8 / 12.4, 128x64x64 30.8 / 25.7, 192x96x96 73.7 / 70.6, 256x128x128 213 /
+// 198, 320x160x160 472 / 388).  16-bit grids between the latency-bound ones and
+// those well beyond the cache are staged (staged / in place, MB of the grid):
+//   FP16   26: 25.2 / 23.3   45: 33.7 / 33.3   51: 35.0 / 35.6   75: 42.1 / 44.8
+//         226: 94.7 / 102.9 283: 158 / 168    321: 187.2 / 189.1 341: 196.9 / 196.3
+//         362: 209 / 203    422: 246 / 228    601: 366 / 329
+//   BF16   26: 24.0 / 21.7   45: 33.5 / 32.7   51: 34.6 / 35.6   75: 42.4 / 44.3
+//         226: 94.8 / 102.4 283: 159.9 / 163.5 301: 176.7 / 175.0 321: 189.1 / 184.8
+//         362: 210 / 198    422: 246 / 222    601: 366 / 324
+constexpr size_t STAGE_FROM = (size_t)48 << 20;
+constexpr size_t STAGE_TO_F16 = (size_t)336 << 20, STAGE_TO_BF16 = (size_t)288 << 20;
 static int listed_mode(const psl_grid* g) {
   const size_t bytes = 27ull * ncells(g) * storage_bytes(g->storage);
   if (g->storage == PSL_F32) return LIST_INLINE;
-  // a level with a finer one inside finds the cache swept by it (two-level FP16
-  // sphere, per coarse step: 770 us staged, 765 in place)
+  // a level with a finer one inside finds the cache swept by it (two-level sphere,
+  // us per coarse step, staged / in place at coarse levels of 91, 145, 216, 308 and
+  // 422 MB: FP16 350.3 / 349.2, 530.2 / 526.6, 774 / 769, 1071 / 1061, 1437 / 1411,
+  // BF16 345.8 / 341.1, 529.5 / 523.0, 776 / 768, 1071 / 1055, 1442 / 1410)
   if (has_subgrid(g->info)) return LIST_INLINE;
-  return bytes < ((size_t)64 << 20) || bytes > ((size_t)256 << 20) ? LIST_INLINE : LIST_STAGE;
+  const size_t to = g->storage == PSL_F16DEV ? STAGE_TO_F16 : STAGE_TO_BF16;
+  return bytes < STAGE_FROM || bytes > to ? LIST_INLINE : LIST_STAGE;
 }
 
 static Faces faces_of(const psl_grid* g) {

@@ -56,9 +56,11 @@ def test_copies_inside_a_call_equal_copy_passes(psl, storage, copies):
         b.close()
 
 
-# FP16 / BF16: 69 MB is staged; 21 MB and 286 MB, and every FP32 grid, are updated in place
+# FP16 / BF16 grids of 66 MB are staged, and FP16 ones of 274 MB; 20 MB, BF16 of 307 MB, FP16 of
+# 356 MB, and every FP32 grid, are updated in place
 @pytest.mark.parametrize("storage,shape", [("f16", (128, 100, 100)), ("bf16", (130, 99, 101)), ("f16", (74, 73, 72)),
-                                           ("f16", (260, 145, 141)), ("f32", (131, 70, 69))])
+                                           ("f16", (260, 145, 141)), ("f32", (131, 70, 69)), ("f16", (300, 151, 153)),
+                                           ("bf16", (287, 145, 143))])
 def test_box_faces_staged_and_in_place_equal_the_fused_launch(psl, storage, shape):
     P = psl
     rng = np.random.default_rng(3)
