@@ -798,9 +798,9 @@ static int periodic_copy(psl_grid* g, int axis) {
   return PSL_OK;
 }
 
-// Whether a call's steps pass the periodic copies on through the ring: the
-// rings exist, every cell is updated (a skipped cell leaves what it holds in
-// its slots, which only a copy pass sees) and the x faces are copied.  An x
+// Whether a call's steps pass the periodic copies on through the ring: every
+// cell is updated (a skipped cell leaves what it holds in its slots, which only
+// a copy pass sees) and the x faces are copied.  An x
 // copy moves one word per line (70 us per step on FP16 257x257x256, 2-4 us and
 // a launch on small grids), and through the ring costs the update 4 %; y
 // copies alone are contiguous passes of 5-10 us, no more than what the ring
@@ -813,12 +813,13 @@ static int periodic_copy(psl_grid* g, int axis) {
 // 17x17x16 12.4 / 13.7, 33x33x32 12.9 / 12.4, 65x65x64 19.2 / 15.3).
 constexpr uint32_t RING_CELLS = 32768;
 static bool ring_runs(const psl_grid* g) {
-  return g->ring_x && !g->census[2] && !g->closure && !(g->flags && g->n_bc);
+  return (g->periodic_copies & 1) && g->info.cellCountX > 1 && ncells(g) >= RING_CELLS && !g->census[2] &&
+         !g->closure && !(g->flags && g->n_bc);
 }
 
-// The rings of the grid's copied faces, made when a call first has two steps;
+// The rings of the grid's copied faces, made when a call first uses them;
 // without them (no memory, or a capture going on) the steps use copy passes.
-static void ensure_rings(psl_grid* g) {
+static bool ensure_rings(psl_grid* g) {
   const psl_info& I = g->info;
   const size_t esz = storage_bytes(g->storage);
   auto make = [&](void** p, size_t bytes) {
@@ -832,18 +833,11 @@ static void ensure_rings(psl_grid* g) {
     return false;
   };
   const bool y = (g->periodic_copies & 2) && I.cellCountY > 1;
-  if (y && !make(&g->ring_y, 4 * 9 * (size_t)I.cellCountX * I.cellCountZ * esz)) return;
-  (void)make(&g->ring_x, 4 * (size_t)I.cellCountY * I.cellCountZ * X_RUN * esz);
+  return (!y || make(&g->ring_y, 4 * 9 * (size_t)I.cellCountX * I.cellCountZ * esz)) &&
+         make(&g->ring_x, 4 * (size_t)I.cellCountY * I.cellCountZ * X_RUN * esz);
 }
-
 int grid_steps(psl_grid* g, int steps) {
-  bool ring = false;
-  if (steps > 1 && (g->periodic_copies & 1) && g->info.cellCountX > 1 && ncells(g) >= RING_CELLS) {
-    ensure_rings(g);
-    ring = ring_runs(g);
-    // y copies of more than a layer need their ring too
-    if ((g->periodic_copies & 2) && g->info.cellCountY > 1 && !g->ring_y) ring = false;
-  }
+  const bool ring = steps > 1 && ring_runs(g) && ensure_rings(g);
   CopyStep c{0u, false, false};
   for (int s = 0; s < steps; ++s) {
     int rc = psl_apply_streaming(g);

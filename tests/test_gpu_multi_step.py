@@ -1,6 +1,8 @@
 """Calls of several steps (psl_update_grid) against the same steps one call at a
 time: the periodic copies passed on inside the update, and the box-face cells
 updated in the bulk kernel or staged, leave the same bits in every cell."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -54,6 +56,32 @@ def test_copies_inside_a_call_equal_copy_passes(psl, storage, copies):
             _same(a, b, f"{shape} after {steps}")
         a.close()
         b.close()
+
+
+def test_no_ring_memory_where_the_copies_stay_passes(psl):
+    """A ring of 64 MB for the x copies is made by the first call that uses it, not
+    for a grid with listed cells, whose copies stay passes."""
+    P = psl
+
+    def free():
+        P.synchronize()
+        f, total = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert P.lib().hipMemGetInfo(ctypes.byref(f), ctypes.byref(total)) == 0  # of the runtime psl is linked to
+        return f.value
+
+    shape = (4, 512, 512)
+    n = shape[0] * shape[1] * shape[2]
+    flags = np.zeros(n, np.uint8)
+    flags[: shape[0] * shape[1]] = cases.GIVEN_U | cases.PERIODIC_X | cases.PERIODIC_Y  # listed z face
+    for listed in (True, False):
+        g = _grid(P, shape, "f32", (True, False), 1, flags if listed else None)
+        P.updateGrid([g], 1)
+        before = free()
+        P.updateGrid([g], 2)
+        used = before - free()
+        print(f"  listed {listed}: {used / 2**20:.1f} MB more", flush=True)
+        assert used < 16 << 20 if listed else used >= 64 << 20
+        g.close()
 
 
 # FP16 / BF16 grids of 66 MB are staged, and FP16 ones of 274 MB; 20 MB, BF16 of 307 MB, FP16 of
