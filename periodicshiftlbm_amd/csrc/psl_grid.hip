@@ -825,9 +825,15 @@ static bool ensure_rings(psl_grid* g) {
   auto make = [&](void** p, size_t bytes) {
     if (*p) return true;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(g->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
-        hipMalloc(p, bytes) == hipSuccess)
-      return true;
+    if (hipStreamIsCapturing(g->stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) {
+      // relaxed: in the default mode an allocation invalidates a capture that
+      // another thread has going on on a stream of its own
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+      const bool ok = hipMalloc(p, bytes) == hipSuccess;
+      if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+      if (ok) return true;
+    }
     *p = nullptr;
     (void)hipGetLastError();
     return false;

@@ -2,6 +2,7 @@
 time: the periodic copies passed on inside the update, and the box-face cells
 updated in the bulk kernel or staged, leave the same bits in every cell."""
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -82,6 +83,53 @@ def test_no_ring_memory_where_the_copies_stay_passes(psl):
         print(f"  listed {listed}: {used / 2**20:.1f} MB more", flush=True)
         assert used < 16 << 20 if listed else used >= 64 << 20
         g.close()
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])  # global, thread-local, relaxed
+def test_first_ring_call_leaves_another_threads_capture_valid(psl, mode):
+    """The rings are allocated inside the first call of several steps; a capture that
+    another thread has begun on a stream of its own still ends well, and so does
+    the call."""
+    P = psl
+    hip = P.lib()  # symbols of the runtime psl is linked to
+    streams = [ctypes.c_void_p() for _ in range(2)]
+    for s in streams:
+        assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0
+    a, b = (_grid(P, (65, 41, 40), "f32", (True, True), 1) for _ in range(2))
+    for g in (a, b):
+        P.synchronize()
+        g.set_stream(streams[0].value)
+        P.updateGrid([g], 1)
+    P.synchronize()
+    begun, stepped, rc = threading.Event(), threading.Event(), []
+
+    def capture():
+        graph = ctypes.c_void_p()
+        rc.append(hip.hipStreamBeginCapture(streams[1], mode))
+        begun.set()
+        stepped.wait(60)
+        rc.append(hip.hipStreamEndCapture(streams[1], ctypes.byref(graph)))
+        if graph:
+            hip.hipGraphDestroy(graph)
+
+    t = threading.Thread(target=capture)
+    t.start()
+    begun.wait(60)
+    try:
+        P.updateGrid([a], 4)
+    finally:
+        stepped.set()
+        t.join()
+    P.synchronize()
+    assert rc == [0, 0]
+    for _ in range(4):
+        P.updateGrid([b], 1)
+    P.synchronize()
+    _same(a, b, f"capture mode {mode}")
+    for g in (a, b):
+        g.close()
+    for s in streams:
+        hip.hipStreamDestroy(s)
 
 
 # FP16 / BF16 grids of 66 MB are staged, and FP16 ones of 274 MB; 20 MB, BF16 of 307 MB, FP16 of
