@@ -800,21 +800,37 @@ static int periodic_copy(psl_grid* g, int axis) {
 
 // Whether a call's steps pass the periodic copies on through the ring: every
 // cell is updated (a skipped cell leaves what it holds in its slots, which only
-// a copy pass sees) and the x faces are copied.  An x
-// copy moves one word per line (70 us per step on FP16 257x257x256, 2-4 us and
-// a launch on small grids), and through the ring costs the update 4 %; y
-// copies alone are contiguous passes of 5-10 us, no more than what the ring
-// costs the update (sphere channel 256x128x128 FP32: 198.8 us per step with
-// passes, 198.7 with the ring; 320x160x160 388 / 394).  Listed cells and the
-// learned closure keep the passes: their kernels have no registers to spare
-// (22 VGPR spills with the ring).
-// Grids under RING_CELLS keep them too: their step is bound by latency, most of
-// it fetching the kernels' instructions (us per step, passes against ring: FP16
-// 17x17x16 12.4 / 13.7, 33x33x32 12.9 / 12.4, 65x65x64 19.2 / 15.3).
-constexpr uint32_t RING_CELLS = 32768;
+// a copy pass sees) and the x faces are copied.  An x copy moves one word per
+// line (70 us per step on FP16 257x257x256, 2-4 us and a launch on small grids),
+// and through the ring costs the update 4 %; y copies alone are contiguous
+// passes of 5-10 us, no more than what the ring costs the update (sphere channel
+// 256x128x128 FP32: 198.8 us per step with passes, 198.7 with the ring;
+// 320x160x160 388 / 394).  Listed cells and the learned closure keep the passes:
+// with the ring their kernels spill in the bulk branch (FP16 staged 256x128x128
+// 91 -> 110 us per step), which the in-place FP32 kernel does not (its 20 spilled
+// VGPRs are the boundary branch's; with the ring 22, 388 -> 394 us).
+//
+// The sizes (us per step of a cubic box, passes / ring; x: no y copies):
+//   a small step is bound by latency, most of it fetching the kernels'
+//   instructions: FP32 33x33x32 12.9 / 12.4, 41x41x40 14.0 / 12.9, FP16 17x17x16
+//   12.4 / 13.7, 33x33x32 12.9 / 13.1, 41x41x40 13.6 / 13.5, 49x49x48 14.7 / 13.7, x
+//   37x36x36 10.6 / 11.1, 41x40x40 11.3 / 11.4, 45x44x44 11.8 / 11.6;
+//   FP16 x in the cache, bound by VALU issue: 60 MB 30.4 / 29.2, 74 34.1 / 34.7,
+//   110 44.3 / 45.6, 156 57.4 / 57.8, 214 74.1 / 73.1 (BF16 x 35.2 / 34.8, 46.5 /
+//   45.8, 61.0 / 58.7; with y copies FP16 36.8 / 35.8, 46.8 / 46.8, 60.4 / 59.8);
+//   FP32 just beyond the cache: 219 MB 85.7 / 82.1, 263 131 / 135, 312 145 / 149,
+//   366 177 / 184, 427 208.0 / 209.1, 460 234 / 231, 530 281 / 269, 737 393 / 362.
+constexpr uint32_t RING_CELLS = 32768, RING_CELLS_16BIT = 70000;
+static bool ring_pays(const psl_grid* g) {
+  const uint32_t n = ncells(g);
+  const size_t mb = (27ull * n * storage_bytes(g->storage)) >> 20;
+  if (g->storage == PSL_F32) return n >= RING_CELLS && (mb < 240 || mb >= 448);
+  const bool y = (g->periodic_copies & 2) && g->info.cellCountY > 1;
+  return n >= RING_CELLS_16BIT && (y || g->storage == PSL_BF16DEV || mb < 64 || mb >= 192);
+}
 static bool ring_runs(const psl_grid* g) {
-  return (g->periodic_copies & 1) && g->info.cellCountX > 1 && ncells(g) >= RING_CELLS && !g->census[2] &&
-         !g->closure && !(g->flags && g->n_bc);
+  return (g->periodic_copies & 1) && g->info.cellCountX > 1 && !g->census[2] && !g->closure &&
+         !(g->flags && g->n_bc) && ring_pays(g);
 }
 
 // The rings of the grid's copied faces, made when a call first uses them;

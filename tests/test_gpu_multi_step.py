@@ -33,18 +33,20 @@ def _same(a, b, what):
     assert nbad == 0, f"{what}: {nbad} values differ"
 
 
-# (from 32768 cells on) rows shorter than, equal to and longer than a wave and a
+# (from 32768 cells on, FP32; 16-bit grids from 70000 on) rows shorter than, equal to and longer than a wave and a
 # workgroup; single and double layers on every axis, where a copied face is its
 # own or its neighbour's
 SHAPES = [(2, 130, 128), (3, 200, 60), (5, 100, 70), (17, 50, 41), (63, 3, 180), (64, 4, 130), (65, 5, 110),
           (130, 2, 130), (257, 9, 15), (300, 1, 112), (2, 1, 20000), (17000, 2, 1), (40000, 1, 1)]
+SHAPES_16BIT = [(2, 300, 140), (3, 300, 100), (5, 150, 120), (17, 70, 70), (63, 5, 270), (64, 4, 330), (65, 5, 260),
+                (130, 2, 330), (257, 18, 19), (300, 1, 280), (2, 1, 45000), (45000, 2, 1), (90000, 1, 1)]
 
 
 @pytest.mark.parametrize("storage", ["f32", "f16", "bf16"])
 @pytest.mark.parametrize("copies", [(True, False), (True, True)])
 def test_copies_inside_a_call_equal_copy_passes(psl, storage, copies):
     P = psl
-    for s, shape in enumerate(SHAPES):
+    for s, shape in enumerate(SHAPES + (SHAPES_16BIT if storage != "f32" else [])):
         n = shape[0] * shape[1] * shape[2]
         solid = None
         if s % 3 == 2:  # bounceback cells, on the copied faces too
