@@ -264,14 +264,15 @@ int psl_grid_check_health(psl_grid* grid, int64_t* bad_cells, double* rho_min, d
  * reference steps one grid at a time).  Each grid keeps its own flags, given
  * values, Cs (uniform or per cell) and storage (all grids share the storage);
  * one step of all grids is one bulk launch over the blocks of every grid and
- * (FP16) one launch over all boundary lists, or one fused launch.  Steps are captured
- * in hipGraphs of one step and of steps_per_graph steps (default 1000) and
- * replayed, so nsteps steps take nsteps / steps_per_graph + nsteps %
+ * (FP16) one launch over all boundary lists, or one fused launch.  Steps are
+ * captured in hipGraphs of one step and of steps_per_graph steps (default 1000)
+ * and replayed, so nsteps steps take nsteps / steps_per_graph + nsteps %
  * steps_per_graph graph launches; a batch whose distributions exceed 192 MB
- * instead takes calls of several steps in groups of grids that fit the
- * last-level cache, all steps of one group after the other, launched without
- * a graph.  Every
- * grid's result is bit-identical to stepping it alone.  Grids need flags and
+ * instead takes calls of several steps (from 2, 4 or 6 on, by storage and
+ * variant) in groups of grids that fit the last-level cache, all steps of one
+ * group after the other, launched without a graph.  Every grid's result is
+ * bit-identical to stepping it alone.  After a launch error every grid's
+ * shifter stands at the steps launched for it.  Grids need flags and
  * must not use periodic copies, sub-grids or a learned closure (checked at
  * every psl_batch_step).  The grids' own handles stay valid (get_f,
  * reductions, single-grid steps); changes to a grid's flags, values, nu or Cs
@@ -282,7 +283,7 @@ int psl_batch_create(psl_grid* const* grids, int count, psl_batch** out);
 int psl_batch_destroy(psl_batch* batch);
 int psl_batch_step(psl_batch* batch, int nsteps);
 /* Steps captured in the multi-step graph, 1 .. PSL_BATCH_MAX_STEPS_PER_GRAPH (1: one
- * graph launch per step). */
+ * graph launch per step); calls stepped in groups use no graph. */
 #define PSL_BATCH_MAX_STEPS_PER_GRAPH 10000
 int psl_batch_set_steps_per_graph(psl_batch* batch, int steps);
 int psl_batch_get_steps_per_graph(const psl_batch* batch, int* steps);

@@ -25,7 +25,7 @@
 // than the last-level cache runs in groups of grids that fit it together: each
 // group takes all the steps of the call before the next one starts (grids are
 // independent), and its populations then come from the cache in every step but
-// the first.  A batch that fits, or a call of one step, runs all grids in each
+// the first.  A batch that fits, or a call of few steps, runs all grids in each
 // launch, from hipGraphs: one of a single step and one of steps_per_graph
 // (default 1000) consecutive steps.  The block order of the grids (as given, or largest
 // first) and the kernel variant are chosen by psl_batch_autotune, and with
@@ -249,9 +249,37 @@ void free_batch_device(psl_batch* b) {
 
 // Whether the two-launch form updates the box-face cells in the bulk launch
 // (each in its own lane, as listed_mode of psl_grid.hip does) instead of from
-// the lists: ms per step of 60 channels, lists against in place, FP32 1.955 /
-// 1.760, BF16 1.106 / 1.082, FP16 1.088 / 1.106 (bound by VALU issue in the cache).
+// the lists: us per step, lists / in place,
+//   FP32 4 channels of 0.9 MB 18.3 / 9.9, 16 of 7 MB 60.5 / 43.2, 8 of 23 MB 85.1 /
+//   67.9, 60 of 73 MB on average 1960 / 1769;
+//   BF16 4 of 0.4 MB 18.0 / 11.7, 16 of 3 MB 45.9 / 38.7, 16 of 11 MB 111 / 97.5,
+//   60 of 37 MB 1109 / 1088;
+//   FP16 60 of 37 MB 1065 / 1116 (bound by VALU issue in the cache).
 bool lists_in_place(const psl_batch* b) { return b->storage != PSL_F16DEV; }
+bool fused_form(const psl_batch* b) { return (b->tuning & PSL_TUNE_FUSED_BOUNDARY) && b->total_bnd; }
+
+// Where groups of grids pay: `steps` is the shortest call that steps a batch in
+// groups, and neighbouring grids above `lone` bytes, which would only come from
+// memory one after the other, form one group (groups' gain over every grid in
+// each launch, by steps of the call; 4 grids of the given MB each):
+//   16 bits fused: 60 channels 0.91 at 2 steps, 0.97 / 1.00 / 1.04 / 1.13 at 3 / 4 /
+//   6 / 20; 226 MB 0.97 at 2, 1.06 at 20; 271 MB 0.95, 421 MB 0.96, 562 MB 0.98;
+//   BF16 in place: 60 channels 0.95 / 1.01 / 1.04 / 1.15 at 2 / 3 / 4 / 20; 226 MB
+//   1.04 at 20, 271 MB 0.93, 421 MB 0.97;
+//   FP32 (both forms within 0.03): 60 channels 0.97 / 1.02 / 1.04 / 1.09 at 2 / 3 /
+//   4 / 20; 274 MB 1.06 at 20, 321 MB 1.03, 374 MB 0.99, 432 MB 0.96;
+//   FP16 with lists gains at every length and size, the lists find their grid's
+//   lines again: 60 channels 1.13 / 1.35 at 2 / 20; 271 MB 1.06, 562 MB 1.04.
+struct GroupRule {
+  int steps;
+  size_t lone;
+};
+GroupRule group_rule(const psl_batch* b) {
+  const size_t mb = (size_t)1 << 20;
+  if (b->storage == PSL_F32) return {4, 348 * mb};
+  if (fused_form(b)) return {6, 248 * mb};
+  return lists_in_place(b) || !b->total_bnd ? GroupRule{4, 248 * mb} : GroupRule{2, SIZE_MAX};
+}
 
 // Step s of a run of `steps` steps of one group of grids.
 template <class St>
@@ -261,7 +289,7 @@ int enqueue_step(psl_batch* b, const BatchGroup& G, int s, int steps) {
   if (s == 0)
     k_batch_advance<St><<<(G.ndom * 27 + 255) / 256, 256, 0, b->stream>>>(
         b->d_params, b->d_fbase, b->d_delta, b->d_shift, b->d_dom + G.dom0, (int)G.ndom);
-  const bool fused = (b->tuning & PSL_TUNE_FUSED_BOUNDARY) && b->total_bnd;
+  const bool fused = fused_form(b);
   const bool inl = lists_in_place(b);
   const uint32_t nb = fused ? G.nfused : G.ntile;
   const uint32_t launch = s + 1 < steps ? nb + 1 : nb;
@@ -400,7 +428,11 @@ int build_batch(psl_batch* b) {
   std::vector<int> delta((size_t)nd * 27);
   std::vector<uint32_t> block_domain, block_tile, bblock_domain, bblock_first(nd);
   b->total_cells = 0;
-  b->total_bnd = 0;
+  b->total_bnd = 0;  // (fused_form and group_rule read it)
+  for (const psl_grid* g : b->grids) {
+    b->total_cells += g->info.cellCount;
+    b->total_bnd += g->n_bc;
+  }
   // bulk tiles of 256 * cpt cells: each grid's in turn, or round-robin
   // across the grids (tile t of every grid that has one, then t + 1)
   const uint64_t tile_cells = 256ull * (uint64_t)b->cpt;
@@ -413,7 +445,7 @@ int build_batch(psl_batch* b) {
   b->launch_order.assign(order.begin(), order.end());
   std::vector<size_t> bytes;
   for (int d : order) bytes.push_back((size_t)b->grids[d]->info.cellCount * 27 * storage_bytes(b->storage));
-  const std::vector<size_t> ends = group_ends(bytes, GROUP_BYTES);
+  const std::vector<size_t> ends = group_ends(bytes, GROUP_BYTES, group_rule(b).lone);
   std::vector<BatchEntry> fused;
   size_t at0 = 0;
   b->groups.clear();
@@ -466,8 +498,6 @@ int build_batch(psl_batch* b) {
                      make_fast_div((uint32_t)g->info.cellCountY), (uint32_t)g->info.cellCountZ, g->bc_dev};
     for (int q = 0; q < 27; ++q)
       delta[(size_t)d * 27 + q] = CX[q] + g->info.cellCountX * CY[q] + g->info.cellCountX * g->info.cellCountY * CZ[q];
-    b->total_bnd += g->n_bc;
-    b->total_cells += g->info.cellCount;
   }
   b->whole = BatchGroup{};
   b->whole.ndom = (uint32_t)nd;
@@ -599,8 +629,8 @@ int psl_batch_step(psl_batch* b, int nsteps) {
   if (rc) return rc;
   // a batch beyond the cache: every group of grids runs all its steps in turn,
   // launched as they are (a group's launches are long enough to hide their own
-  // enqueueing); one step of everything gains nothing from groups
-  if (nsteps > 1 && b->groups.size() > 1)
+  // enqueueing); a call of few steps gains nothing from groups
+  if (nsteps >= group_rule(b).steps && b->groups.size() > 1)
     return run_groups(
         b->groups.size(), nsteps, [&](size_t g, int s) { return enqueue_dispatch(b, b->groups[g], s, nsteps); },
         [&](size_t g, int n) { advance_shifters(b, b->groups[g], n); });

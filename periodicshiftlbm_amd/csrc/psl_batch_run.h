@@ -11,12 +11,15 @@ namespace psl {
 // each: grids of `bytes` in turn, as many as fit `limit` together, the groups
 // of a run of them about equal in size.  A grid above `limit` is a group of its
 // own and ends the run, so that its size does not count in the shares of the
-// others.
-inline std::vector<size_t> group_ends(const std::vector<size_t>& bytes, size_t limit) {
+// others; neighbours above `lone` (at least `limit`) are one group.
+inline std::vector<size_t> group_ends(const std::vector<size_t>& bytes, size_t limit, size_t lone) {
   std::vector<size_t> ends;
   for (size_t at = 0; at < bytes.size();) {
     if (bytes[at] > limit) {
-      ends.push_back(++at);
+      const bool together = bytes[at] > lone;
+      do ++at;
+      while (together && at < bytes.size() && bytes[at] > lone);
+      ends.push_back(at);
       continue;
     }
     size_t end = at, total = 0;

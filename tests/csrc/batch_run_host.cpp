@@ -3,8 +3,9 @@
 #include "../../periodicshiftlbm_amd/csrc/psl_batch_run.h"
 
 extern "C" {
-int br_ends(int n, const long long* bytes, long long limit, int* ends) {
-  const std::vector<size_t> e = psl::group_ends(std::vector<size_t>(bytes, bytes + n), (size_t)limit);
+int br_ends(int n, const long long* bytes, long long limit, long long lone, int* ends) {
+  const std::vector<size_t> e = psl::group_ends(std::vector<size_t>(bytes, bytes + n), (size_t)limit,
+                                                    (size_t)lone);
   for (size_t i = 0; i < e.size(); ++i) ends[i] = (int)e[i];
   return (int)e.size();
 }

@@ -45,10 +45,10 @@ def test_graph_shifters_follow_the_launched_steps(host, steps, many, fail, want)
     assert launched.value == moved.value == want
 
 
-def _ends(host, sizes, limit):
+def _ends(host, sizes, limit, lone=1 << 60):
     b, out = np.array(sizes, np.int64), np.zeros(len(sizes), np.int32)
     n = host.br_ends(len(sizes), b.ctypes.data_as(ctypes.c_void_p), ctypes.c_longlong(limit),
-                     out.ctypes.data_as(ctypes.c_void_p))
+                     ctypes.c_longlong(lone), out.ctypes.data_as(ctypes.c_void_p))
     return out[:n].tolist()
 
 
@@ -73,3 +73,10 @@ def test_groups_fill_the_limit(host, seed):
     for a, b in zip(groups, groups[1:]):
         if max(a + b) <= limit:
             assert max(sum(a), sum(b)) > limit // 4
+
+
+def test_neighbours_beyond_the_cache_are_one_group(host):
+    sizes = [400, 500, 10, 20, 250, 300, 401, 5]
+    assert _ends(host, sizes, 192, 350) == [2, 4, 5, 6, 7, 8]
+    assert _ends(host, sizes, 192, 249) == [2, 4, 7, 8]
+    assert _ends(host, [400, 500, 600], 192, 350) == [3]
