@@ -194,8 +194,7 @@ int psl_device_download(void* dst_host, const void* src_device, size_t bytes);
 /* Local-update variants (bits): non-temporal loads / stores and XCD-contiguous
  * block order in the bulk kernel; FUSED_BOUNDARY updates the box-face list by
  * workgroups of its own between the bulk's.  Without it the bulk kernel updates
- * those cells in place or stages them for a second launch, by storage and size;
- * the non-temporal bits apply where it stages them or there are none. */
+ * those cells in place or stages them for a second launch, by storage and size. */
 enum {
   PSL_TUNE_NT_LOAD = 1,
   PSL_TUNE_NT_STORE = 2,

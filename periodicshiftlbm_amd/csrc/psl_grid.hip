@@ -517,42 +517,34 @@ static void drop_profile_events(psl_grid* g) {
   g->prof_events.clear();
 }
 
-// The bulk launch.  Non-temporal variants exist for the plain step only (not
-// with copies through the ring, box-face cells in place or a held closure).
-template <class St>
-static void launch_bulk(int nt, bool flags, bool les, bool held, int list, bool copy, uint32_t nb, size_t lds,
+// The bulk launch.  FP32 box faces are staged on held closure steps only
+// (listed_mode).
+template <class St, int TUNE>
+static void launch_bulk(bool flags, bool les, bool held, int list, bool copy, uint32_t nb, size_t lds,
                         hipStream_t stream, const StepParams& p, const Stage& sg, const Faces& fc,
                         const CopyStep& cs) {
-#define PSL_BULK(F, L, V, M, H, C) k_ps_bulk<St, F, L, V, M, H, C><<<nb, 256, lds, stream>>>(p, sg, fc, cs)
-#define PSL_BULK_LES(F, V, M, C)                  \
-  do {                                            \
-    if (les) PSL_BULK(F, true, V, M, false, C);   \
-    else PSL_BULK(F, false, V, M, false, C);      \
+  constexpr bool F32 = std::is_same<St, StF32>::value;
+#define PSL_BULK(F, L, M, H, C) k_ps_bulk<St, F, L, TUNE, M, H, C><<<nb, 256, lds, stream>>>(p, sg, fc, cs)
+#define PSL_BULK_LES(F, M, C)                  \
+  do {                                         \
+    if (les) PSL_BULK(F, true, M, false, C);   \
+    else PSL_BULK(F, false, M, false, C);      \
   } while (0)
   if (held) {
     // between learned-closure evaluations
-    if (list == LIST_STAGE) PSL_BULK(true, true, 0, LIST_STAGE, true, false);
-    else if (flags) PSL_BULK(true, true, 0, LIST_NONE, true, false);
-    else PSL_BULK(false, true, 0, LIST_NONE, true, false);
+    if (list == LIST_STAGE) PSL_BULK(true, true, LIST_STAGE, true, false);
+    else if (flags) PSL_BULK(true, true, LIST_NONE, true, false);
+    else PSL_BULK(false, true, LIST_NONE, true, false);
   } else if (list == LIST_INLINE) {
-    PSL_BULK_LES(true, 0, LIST_INLINE, false);
+    PSL_BULK_LES(true, LIST_INLINE, false);
+  } else if (list == LIST_STAGE) {
+    if constexpr (!F32) PSL_BULK_LES(true, LIST_STAGE, false);
   } else if (copy) {
-    if (flags) PSL_BULK_LES(true, 0, LIST_NONE, true);
-    else PSL_BULK_LES(false, 0, LIST_NONE, true);
+    if (flags) PSL_BULK_LES(true, LIST_NONE, true);
+    else PSL_BULK_LES(false, LIST_NONE, true);
   } else {
-#define PSL_BULK_V(V)                                            \
-  case V:                                                        \
-    if (list == LIST_STAGE) PSL_BULK_LES(true, V, LIST_STAGE, false); \
-    else if (flags) PSL_BULK_LES(true, V, LIST_NONE, false);     \
-    else PSL_BULK_LES(false, V, LIST_NONE, false);               \
-    break
-    switch (nt) {
-      PSL_BULK_V(0);
-      PSL_BULK_V(1);
-      PSL_BULK_V(2);
-      PSL_BULK_V(3);
-    }
-#undef PSL_BULK_V
+    if (flags) PSL_BULK_LES(true, LIST_NONE, false);
+    else PSL_BULK_LES(false, LIST_NONE, false);
   }
 #undef PSL_BULK_LES
 #undef PSL_BULK
@@ -692,8 +684,14 @@ static int launch_local_update(psl_grid* g, bool dominant_only = false, const Co
       default: launch_fused<St, 3>(les, nf, g->stream, p, b, g->fused_dev); break;
     }
   } else {
-    launch_bulk<St>(nt, g->flags != nullptr, les, held, list, copy, nb, g->bulk_lds, g->stream, p,
-                    Stage{list == LIST_STAGE ? g->stage_buf : nullptr, g->stage_base}, fc, cstep);
+    const bool fl = g->flags != nullptr;
+    const Stage sg{list == LIST_STAGE ? g->stage_buf : nullptr, g->stage_base};
+    switch (nt) {
+      case 0: launch_bulk<St, 0>(fl, les, held, list, copy, nb, g->bulk_lds, g->stream, p, sg, fc, cstep); break;
+      case 1: launch_bulk<St, 1>(fl, les, held, list, copy, nb, g->bulk_lds, g->stream, p, sg, fc, cstep); break;
+      case 2: launch_bulk<St, 2>(fl, les, held, list, copy, nb, g->bulk_lds, g->stream, p, sg, fc, cstep); break;
+      default: launch_bulk<St, 3>(fl, les, held, list, copy, nb, g->bulk_lds, g->stream, p, sg, fc, cstep); break;
+    }
   }
   PSL_LAUNCH_CHECK();
   if (g->profile) {

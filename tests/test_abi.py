@@ -34,6 +34,22 @@ def test_abi_version_and_error_path_without_gpu():
     assert b"null" in L.psl_last_error()
 
 
+def test_every_bulk_kernel_has_its_non_temporal_variants():
+    """The non-temporal tuning bits reach every form of the bulk kernel: plain,
+    staging, in place, held closure and copies through the ring (the kernels'
+    names in the library: storage, FLAGS, LES, TUNE, LIST, HELD, COPY)."""
+    import periodicshiftlbm_amd as P
+    data = open(P.LIB_PATH, "rb").read()
+    found = set(re.findall(rb"k_ps_bulkINS_\d+(St\w+?)ELb(\d)ELb(\d)ELi(\d)ELi(\d)ELb(\d)ELb(\d)EE", data))
+    forms = {k[:3] + k[4:] for k in found}
+    assert {(b"StF16", b"1", b"1", b"2", b"0", b"0"), (b"StF16", b"1", b"1", b"1", b"0", b"0"),
+            (b"StF32", b"1", b"1", b"1", b"1", b"0"), (b"StBF16", b"0", b"0", b"0", b"0", b"1")} <= forms
+    missing = [(f, t) for f in forms for t in (b"0", b"1", b"2", b"3") if f[:3] + (t,) + f[3:] not in found]
+    assert not missing, missing
+    # FP32 grids update their box faces in place, staging them on held steps only
+    assert not [f for f in forms if f[0] == b"StF32" and f[3] == b"1" and f[4] == b"0"]
+
+
 def test_oracle_library_is_test_only():
     """The product library does not link the oracle."""
     import periodicshiftlbm_amd as P

@@ -61,6 +61,27 @@ def test_copies_inside_a_call_equal_copy_passes(psl, storage, copies):
         b.close()
 
 
+@pytest.mark.parametrize("storage,shape", [("f32", (65, 41, 40)), ("f16", (65, 36, 35)), ("bf16", (63, 37, 36))])
+@pytest.mark.parametrize("solid", [False, True])
+def test_copies_inside_a_call_at_every_variant(psl, storage, shape, solid):
+    """The non-temporal forms of the update with copies through the ring."""
+    P = psl
+    n = shape[0] * shape[1] * shape[2]
+    flags = None
+    if solid:
+        flags = np.where(np.random.default_rng(3).random(n) < 0.2, cases.BOUNCEBACK, cases.FLUID).astype(np.uint8)
+    b = _grid(P, shape, storage, (True, True), 1, flags)
+    for _ in range(4):
+        P.updateGrid([b], 1)
+    for v in range(P.TUNE_VARIANTS):
+        a = _grid(P, shape, storage, (True, True), 1, flags)
+        a.tuning = v
+        P.updateGrid([a], 4)
+        _same(a, b, f"{storage} {shape} variant {v}")
+        a.close()
+    b.close()
+
+
 def test_no_ring_memory_where_the_copies_stay_passes(psl):
     """A ring of 64 MB for the x copies is made by the first call that uses it, not
     for a grid with listed cells, whose copies stay passes."""
