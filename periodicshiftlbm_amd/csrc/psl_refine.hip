@@ -36,7 +36,7 @@ struct Face {
   uint32_t blocks;
   uint32_t ghost_pops;  // bit q: population q is written to ghost fine cells
 };
-struct Faces {
+struct FaceSet {
   Face f[6];
   int count;
 };
@@ -91,7 +91,7 @@ constexpr int TF_CELLS = 64;  // coarse cells per workgroup, coarse->fine
 template <class St>
 __global__ __launch_bounds__(256) void k_to_coarse(typename St::T* __restrict__ fc, GridView gc, int iss, int jss,
                                                    int kss, const typename St::T* __restrict__ ff, GridView gf,
-                                                   Faces faces) {
+                                                   FaceSet faces) {
   __shared__ float part[4][27][TC_CELLS];
   const Face& F = faces.f[blockIdx.y];
   if (blockIdx.x >= F.blocks) return;
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(256) void k_to_coarse(typename St::T* __restrict__ 
 template <class St>
 __global__ __launch_bounds__(256) void k_to_fine(const typename St::T* __restrict__ fc, GridView gc, int iss, int jss,
                                                  int kss, typename St::T* __restrict__ ff, GridView gf,
-                                                 const uint8_t* __restrict__ fine_flags, Faces faces) {
+                                                 const uint8_t* __restrict__ fine_flags, FaceSet faces) {
   __shared__ float st[4][27][TF_CELLS];
   const Face& F = faces.f[blockIdx.y];
   if (blockIdx.x >= F.blocks) return;
@@ -212,7 +212,7 @@ static GridView view_of(const psl_grid* g) {
 
 // Appends the coarse box [s, e) as a face; the first axis with more than one
 // cell runs along the workgroup.
-static void add_face(Faces& F, const int s[3], const int e[3], int cells_per_block, uint32_t ghost_pops) {
+static void add_face(FaceSet& F, const int s[3], const int e[3], int cells_per_block, uint32_t ghost_pops) {
   int n[3];
   for (int d = 0; d < 3; ++d) n[d] = std::max(0, e[d] - s[d]);
   if (n[0] == 0 || n[1] == 0 || n[2] == 0) return;
@@ -233,7 +233,7 @@ static void add_face(Faces& F, const int s[3], const int e[3], int cells_per_blo
   f.ghost_pops = ghost_pops;
 }
 
-static uint32_t face_blocks(const Faces& F) {
+static uint32_t face_blocks(const FaceSet& F) {
   uint32_t m = 0;
   for (int i = 0; i < F.count; ++i) m = std::max(m, F.f[i].blocks);
   return m;
@@ -253,7 +253,7 @@ static const int POS_Z[9] = {4, 8, 9, 14, 17, 20, 21, 24, 26};
 static const int NEG_Z[9] = {3, 7, 10, 13, 18, 19, 22, 23, 25};
 
 template <class St>
-static int to_coarse(psl_grid* c, psl_grid* f, const Faces& F) {
+static int to_coarse(psl_grid* c, psl_grid* f, const FaceSet& F) {
   const uint32_t nb = face_blocks(F);
   if (nb == 0) return PSL_OK;
   dim3 grid(nb, F.count);
@@ -265,7 +265,7 @@ static int to_coarse(psl_grid* c, psl_grid* f, const Faces& F) {
 }
 
 template <class St>
-static int to_fine(psl_grid* c, psl_grid* f, const Faces& F) {
+static int to_fine(psl_grid* c, psl_grid* f, const FaceSet& F) {
   const uint32_t nb = face_blocks(F);
   if (nb == 0) return PSL_OK;
   dim3 grid(nb, F.count);
@@ -281,7 +281,7 @@ static int communicate(psl_grid* c, psl_grid* f, bool full_fill) {
   const psl_info& C = c->info;
   const int is = C.iSubgridStart, js = C.jSubgridStart, ks = C.kSubgridStart;
   const int ie = C.iSubgridEnd, je = C.jSubgridEnd, ke = C.kSubgridEnd;
-  Faces B{};
+  FaceSet B{};
   if (full_fill) {
     const int s[3] = {is + 1, js + 1, ks + 1}, e[3] = {ie - 1, je - 1, ke - 1};
     add_face(B, s, e, TC_CELLS, 0);
@@ -310,7 +310,7 @@ static int communicate(psl_grid* c, psl_grid* f, bool full_fill) {
   if (rc) return rc;
   // coarse -> fine layers (lines 488-525): two fine cells deep, i.e. one
   // coarse layer of the sub-grid, on each side that is not the grid edge
-  Faces Fb{};
+  FaceSet Fb{};
   auto add = [&](int s0, int s1, int s2, int e0, int e1, int e2, const int(&dirs)[9]) {
     const int s[3] = {s0, s1, s2}, e[3] = {e0, e1, e2};
     add_face(Fb, s, e, TF_CELLS, pop_mask(dirs));

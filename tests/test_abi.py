@@ -50,6 +50,20 @@ def test_every_bulk_kernel_has_its_non_temporal_variants():
     assert not [f for f in forms if f[0] == b"StF32" and f[3] == b"1" and f[4] == b"0"]
 
 
+def test_no_type_name_is_defined_in_two_files():
+    """One definition per type of the library's sources: two of one name in one
+    namespace would let an inline function of one file bind to the other's layout."""
+    src = os.path.join(REPO, "periodicshiftlbm_amd", "csrc")
+    where = {}
+    for name in sorted(os.listdir(src)):
+        if name.endswith((".h", ".hip", ".inc")):
+            text = open(os.path.join(src, name)).read()
+            for t in re.findall(r"^(?:struct|class) (\w+)[^;{]*\{", text, flags=re.M):
+                where.setdefault(t, []).append(name)
+    assert len(where) > 20
+    assert not {t: f for t, f in where.items() if len(f) > 1}
+
+
 def test_oracle_library_is_test_only():
     """The product library does not link the oracle."""
     import periodicshiftlbm_amd as P
