@@ -1,4 +1,4 @@
-"""Seeded random small periodic-shift configurations shared by the GPU tests
+"""Seeded random periodic-shift configurations shared by the GPU tests
 (test_gpu_random_configs, test_gpu_random_batch).
 
 A case is a shape of 2-20 x 1-12 x 1-12 cells, a kind and a given-value slot
@@ -15,12 +15,15 @@ from periodicshiftlbm_amd import cases
 FACE_KINDS = [cases.GIVEN_U, cases.GIVEN_RHO, cases.GIVEN_NONE, cases.GIVEN_RHOU, cases.BOUNCEBACK, cases.FLUID]
 
 
-def config(seed, large=False):
+def config(seed, large=False, staged=False):
     """Small grids (2-20 x 1-12 x 1-12 cells), or with large=True 24-72 cells
-    per axis: many workgroups, wrap thresholds inside waves, several blocks of
-    staged boundary records."""
-    rng = np.random.default_rng((31000 if large else 1000) + seed)
-    if large:
+    per axis: many workgroups, wrap thresholds inside waves, or with staged=True
+    100-127 cells per axis: 16-bit grids of 51 to 106 MB, whose box faces are
+    staged (many blocks of boundary records)."""
+    rng = np.random.default_rng((61000 if staged else 31000 if large else 1000) + seed)
+    if staged:
+        shape = tuple(int(x) for x in rng.integers(100, 128, 3))
+    elif large:
         shape = tuple(int(x) for x in rng.integers(24, 73, 3))
     else:
         shape = (int(rng.integers(2, 21)), int(rng.integers(1, 13)), int(rng.integers(1, 13)))

@@ -133,8 +133,8 @@ def test_batch_autotune_keeps_results(psl):
 
 @pytest.mark.parametrize("storage", ["f32", "f16", "bf16"])
 def test_single_grid_variants_identical(psl, storage):
-    """Every local-update variant of the single-grid path (staged or fused box
-    faces, plain or non-temporal accesses, either block order) gives the same bits."""
+    """Every local-update variant of the single-grid path (box faces in place or
+    fused, plain or non-temporal accesses, either block order) gives the same bits."""
     P = psl
     d = _domains()[1]
     ref = cases.domain_grid(d, storage)[0]

@@ -315,6 +315,65 @@ def test_held_closure_matches_oracle(psl, oracle_mod):
     assert e2_fresh > 10 * e2  # the held update did not evaluate the network
 
 
+@pytest.mark.parametrize("storage", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("shape,tuning", [((48, 24, 24), 4), ((37, 19, 23), 4), ((48, 24, 24), 3)])
+def test_closure_steps_with_box_faces(psl, storage, shape, tuning):
+    """A channel with inlet, outlet and solid cells under a constant network
+    (y0 = 2, exact in FP16), evaluated every third step.  An evaluating step
+    (listed cells from their slots) and a held one (staged) from one state each
+    leave the bits of the step without a closure in the listed and the solid
+    cells (nu and Cs as set), and in the fluid ones the values at nu + 1e-3 y0
+    without Smagorinsky: the viscosities' sums differ by a rounding, so within
+    1e-5 as the other constant-network test, 2 units in the last place of f - w
+    in 16 bits (0.1 x 2^-10 and 0.1 x 2^-7)."""
+    P = psl
+    nx, ny, nz = shape
+    n = nx * ny * nz
+    rng = np.random.default_rng(21)
+    nu, y0 = 0.004, 2.0
+    k, j, i = np.meshgrid(np.arange(nz), np.arange(ny), np.arange(nx), indexing="ij")
+    solid = ((i - 12) ** 2 + (j - 10) ** 2 + (k - 11) ** 2 <= 16).reshape(-1) | (rng.random(n) < 0.05)
+    flags = cases.channel_flags(shape, solid)
+    fill = [rng.uniform(0.98, 1.02, n).astype(np.float32), *rng.uniform(-0.03, 0.03, (3, n)).astype(np.float32)]
+    p = np.zeros(C.N_PARAM, np.float32)
+    p[-1] = y0
+    net = P.MLP(p)
+
+    def grid(nu, cs, closure):
+        g = P.GridStruct(P.InfoStruct(cellCountX=nx, cellCountY=ny, cellCountZ=nz, nu=nu), storage)
+        g.set_flags(flags)
+        g.set_given_values(cases.channel_given_values(0.03))
+        g.set_smagorinsky(cs)
+        g.set_periodic_copies(y=True)
+        g.tuning = tuning
+        P.fill_equilibrium(g, *fill)
+        if closure:
+            g.set_closure(net)
+            g.set_closure_every(3)
+        return g
+
+    kind = flags & 7
+    listed, fluid = (kind >= cases.GIVEN_RHO) & (kind <= cases.GIVEN_RHOU), kind == cases.FLUID
+    assert listed.sum() > 0 and (kind == cases.BOUNCEBACK).sum() > 0
+    bound = {"f32": 1e-5, "f16": 0.2 * 2.0 ** -10, "bf16": 0.2 * 2.0 ** -7}[storage]
+    g, base, shifted = grid(nu, 0.12, True), grid(nu, 0.12, False), grid(nu + C.NU_SCALE * y0, 0.0, False)
+    f0 = g.get_f()
+    for what in ("evaluating", "held", "held"):
+        out = []
+        for x in (g, base, shifted):
+            x.set_f(f0)
+            P.updateGrid([x], 1)
+            out.append(x.get_f())
+        nbad = int(np.count_nonzero(out[0].view(np.uint32)[:, ~fluid] != out[1].view(np.uint32)[:, ~fluid]))
+        err = float(np.max(np.abs(out[0][:, fluid].astype(np.float64) - out[2][:, fluid])))
+        print(f"  {what}: {nbad} listed or solid values differ, fluid {err:.2e}", flush=True)
+        assert nbad == 0
+        assert err < bound
+        f0 = out[1]
+    for x in (g, base, shifted):
+        x.close()
+
+
 def _features_from_f(f):
     """Raw closure features of populations (n, 27) in FP64 (central second moments)."""
     from oracle import velocity_set

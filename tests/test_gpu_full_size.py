@@ -9,7 +9,7 @@ size).
     - 20 steps against the FP32 oracle at full size, 1e-5 relative (the
       oracle's mixed FP32/FP64 expressions), and the momentum-exchange force
       on the sphere box against the oracle's;
-    - every local-update variant (staged or fused box faces, non-temporal
+    - every local-update variant (box faces in place or fused, non-temporal
       loads / stores, block order) ends on the same bits after 20 steps.
 * The same channel from rest over 20000 steps (flowAroundSphereMainSingle.cu
   records C_D every step): with f - w stored in FP16 the mean drag

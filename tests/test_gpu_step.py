@@ -328,7 +328,7 @@ def test_ragged_grids_match_oracle(psl, oracle_mod, shape):
 
 def test_small_channel_with_boundary_cells_matches_oracle(psl, oracle_mod):
     """A 6 x 4 x 3 channel: inlet and outlet faces are most of the grid, so the
-    boundary list and its staged / fused paths carry most cells."""
+    boundary list and its in-place / fused paths carry most cells."""
     P, O = psl, oracle_mod
     shape = (6, 4, 3)
     n = int(np.prod(shape))
