@@ -196,7 +196,7 @@ __global__ __launch_bounds__(256) void k_eso_update(typename St::T* __restrict__
   if (kind == KIND_GHOST || kind == KIND_COVERED) kind = KIND_GIVEN_NONE;
   uint32_t slot[8];
   eso_slots_adj(p, cell, slot);
-  auto at = [&](int row, int s) { return (T*)((char*)(f + (size_t)row * p.n) + (Off)slot[s] * (Off)sizeof(T)); };
+  auto at = [&](int row, int s) { return row_slot<T, Off>(f, row, p.n, slot[s]); };
   Word<St> r[27];
 #pragma unroll
   for (int q = 0; q < 27; ++q) r[q] = (Word<St>)ld<T, false>(at(FLIP ? q : opp(q), ESO_READ[q]));
@@ -1033,7 +1033,7 @@ static int eso_update(psl_diad* d, bool child_records) {
   const EsoParams p = eso_params(d, child_records);
   const uint32_t nb = (uint32_t)((d->n + 255) / 256);
   typename St::T* f = (typename St::T*)d->f;
-  if ((uint64_t)p.n * sizeof(typename St::T) > 0xffffffffull) {
+  if (wide_rows<typename St::T>(p.n)) {
     if (d->flipper) k_eso_update<St, true, true><<<nb, 256, 0, d->stream>>>(f, p);
     else k_eso_update<St, false, true><<<nb, 256, 0, d->stream>>>(f, p);
   } else {

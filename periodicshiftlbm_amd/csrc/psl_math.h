@@ -33,6 +33,7 @@
 // batched) produces the same bits for the same cell.
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 #pragma clang fp contract(on)
@@ -48,6 +49,18 @@
 #endif
 
 namespace psl {
+
+// Word `slot` of a row of n words: the row's base and an offset in bytes, 32 bits
+// wide (Off = uint32_t) where rows are shorter than 4 GiB, so that an access takes
+// its base from scalar registers; wide_rows says where it is not enough.
+template <class T, class Off>
+PSL_HD PSL_INLINE T* row_slot(T* f, int row, uint32_t n, uint32_t slot) {
+  return (T*)((char*)(f + (size_t)row * n) + (Off)slot * (Off)sizeof(T));
+}
+template <class T>
+PSL_HD PSL_INLINE bool wide_rows(uint32_t n) {
+  return (uint64_t)n * sizeof(T) > 0xffffffffull;
+}
 
 // D3Q27 ordering of the reference (include/applyStreaming.h:1-8).
 // id:  0  1  2  3  4  5  6  7  8  9 10 11 12 13 14 15 16 17 18 19 20 21 22 23 24 25 26

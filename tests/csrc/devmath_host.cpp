@@ -3,6 +3,15 @@
 // without a GPU.  Test infrastructure only.
 #include "../../periodicshiftlbm_amd/csrc/psl_math.h"
 
+// Bytes from the first word of a field to word `slot` of `row`, as the esotwist
+// update addresses it.
+template <class T>
+static long long row_offset(int row, unsigned n, unsigned slot) {
+  T* f = (T*)(uintptr_t)4096;
+  T* at = psl::wide_rows<T>(n) ? psl::row_slot<T, size_t>(f, row, n, slot) : psl::row_slot<T, uint32_t>(f, row, n, slot);
+  return (long long)((uintptr_t)at - (uintptr_t)f);
+}
+
 extern "C" {
 void dm_collide(float* f, long long n, float nu, float cs, int w_off) {
   const float tau = 3.f * nu + 0.5f;
@@ -35,6 +44,11 @@ int dm_bc(int which, int code, float* f, float* ru) {
   ru[0] = rho; ru[1] = ux; ru[2] = uy; ru[3] = uz;
   return 0;
 }
+// Words of `bytes` bytes (2 or 4).
+long long dm_row_offset(int bytes, int row, unsigned n, unsigned slot) {
+  return bytes == 2 ? row_offset<uint16_t>(row, n, slot) : row_offset<float>(row, n, slot);
+}
+int dm_wide_rows(int bytes, unsigned n) { return bytes == 2 ? psl::wide_rows<uint16_t>(n) : psl::wide_rows<float>(n); }
 float dm_feq(int q, float rho, float ux, float uy, float uz) { return psl::feq(q, rho, ux, uy, uz); }
 }
 

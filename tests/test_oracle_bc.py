@@ -153,3 +153,17 @@ def test_device_collision_formulation_matches_oracle(devmath):
         devmath.dm_rescale(a.ctypes.data, n, c2f)
         o = O.rescale(f, bool(c2f))
         assert np.max(np.abs(a - o) / np.abs(o)) < 5e-6
+
+
+@pytest.mark.parametrize("size", [2, 4])
+def test_esotwist_row_offsets_around_4_gib(devmath, size):
+    """Words of rows of up to 2^32 bytes and beyond: 32-bit offsets reach every
+    word of a row, and longer rows take 64-bit ones."""
+    devmath.dm_row_offset.restype = ctypes.c_longlong
+    devmath.dm_row_offset.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_uint, ctypes.c_uint]
+    devmath.dm_wide_rows.argtypes = [ctypes.c_int, ctypes.c_uint]
+    for n in (1, 257, (1 << 30) - 1, 1 << 30, (1 << 30) + 1, (1 << 31) - 1):
+        assert devmath.dm_wide_rows(size, n) == (n * size >= 1 << 32)
+        for row in (0, 13, 26):
+            for slot in (0, n // 2, n - 1):
+                assert devmath.dm_row_offset(size, row, n, slot) == (row * n + slot) * size
