@@ -43,7 +43,6 @@ struct EsoParams {
   void* srec;                 // source records
   const uint64_t* srec_mask;
   const uint32_t* srec_base;
-  bool deal4;  // the local update's blocks go to the XCDs four at a time
 };
 
 // Interface records: the post-collision storage words of one cell, in q
@@ -169,25 +168,18 @@ __global__ void k_eso_adjacency(const int* __restrict__ nbr, uint32_t n, uint8_t
 // Bound by the traffic of the 27 populations' rows: 4.45 TB/s of them in FP16 on
 // a dense 256^3 box (41 GLUPS), 3.4 on the sparse levels, whose rows of tens of
 // cells split a wave's stores over many lines.  Two choices follow from the
-// latter: on sparse levels blocks are dealt to the XCDs four at a time (p.deal4),
-// so that the lines at their borders are shared in one L2 (6-level sphere, FP16:
-// 60.6 ms per coarse step one at a time, 59.8 / 60.0 / 60.4 at 4 / 16 / 64, one
-// range per XCD 64; levels of 0.1 to 5 M cells gain 0 to 5 %), and each access is
-// a scalar row base and a 32-bit offset, the populations staying storage words
-// until the moments, which takes 89 VGPRs instead of 114 (61.4 -> 60.6 ms).  Held
-// to 80 or 72 VGPRs it spills (71 and 97 ms).  WIDE: rows of 4 GiB and more.
-//
-// A level that fills its box keeps one block at a time: its planes and rows come
-// at regular distances, and at sizes of a power of two the four-block order puts
-// a cell and its +k neighbour on different XCDs, or several streams on one
-// channel (us per update, one / four at a time: FP16 64^3 8.3 / 10.5, 128^3 43.5
-// / 52.2, 256x128x64 42.0 / 48.9; FP32 64^3 8.7 / 10.3, 192x128x128 140 / 149;
-// other sizes gain up to 9 %, FP16 80^3 14.9 / 14.0, 256^3 404 / 394).
-template <class St, bool FLIP, bool WIDE>
+// latter: blocks are dealt to the XCDs four at a time (DEAL4, where deal4 says
+// so), so that the lines at their borders are shared in one L2 (6-level sphere,
+// FP16: 60.6 ms per coarse step one at a time, 59.8 / 60.0 / 60.4 at 4 / 16 / 64,
+// one range per XCD 64), and each access is a scalar row base and a 32-bit offset,
+// the populations staying storage words until the moments, which takes 87 VGPRs
+// instead of 114 (61.4 -> 60.6 ms).  Held to 80 or 72 VGPRs it spills (71 and 97
+// ms).  WIDE: rows of 4 GiB and more.
+template <class St, bool FLIP, bool WIDE, bool DEAL4>
 __global__ __launch_bounds__(256) void k_eso_update(typename St::T* __restrict__ f, EsoParams p) {
   typedef typename St::T T;
   typedef typename std::conditional<WIDE, size_t, uint32_t>::type Off;
-  const uint32_t block = p.deal4 ? xcd_block_chunked<4>(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint32_t block = DEAL4 ? xcd_block_chunked<4>(blockIdx.x, gridDim.x) : blockIdx.x;
   const uint32_t cell = block * 256u + threadIdx.x;
   if (cell >= p.n) return;
   const int fl = p.flags ? p.flags[cell] : 0;
@@ -881,7 +873,6 @@ static EsoParams eso_params(const psl_diad* d, bool child_records = true) {
   p.srec = d->source.n ? d->source.rec : nullptr;
   p.srec_mask = d->source.mask;
   p.srec_base = d->source.base;
-  p.deal4 = (int64_t)d->n != (int64_t)p.nx * p.ny * p.nz;
   return p;
 }
 
@@ -1028,18 +1019,50 @@ static int diad_prepare_records(psl_diad* const* lv, int nl) {
   return PSL_OK;
 }
 
+// Whether the update's blocks go to the XCDs four at a time: on sparse levels
+// (0.1 to 27 M cells, gain 0 to 5 %) and on most boxes (us per update, one / four
+// at a time: FP16 80^3 15.0 / 13.4, 96^3 22.7 / 21.7, 256^3 404 / 394; FP32 48^3
+// 8.8 / 8.1, 80^3 22.8 / 20.5).  On a box that is full or nearly so planes and rows
+// come at regular distances, and one at a time is better where
+//   the level has less than a block per CU, where neither order gains throughout
+//   (32^3: FP32 4.8 / 4.6, FP16 4.1 / 3.8 to 4.4, BF16 4.1 / 4.5);
+//   the populations stay in the L2s and planes are a multiple of 8 blocks but not
+//   of 32: a cell's +k neighbour is then on its own XCD one at a time, on the
+//   fourth other XCD four at a time (FP16 64^3 8.0 / 10.4, 96x64x64 10.6 / 11.4,
+//   64x65x64 9.1 / 11.2, FP32 64^3 8.3 / 9.9, 64x64x80 12.7 / 13.1);
+//   rows of 4 to 16 MiB are a multiple of 4 MiB: the XCDs' streams meet on the
+//   same channels (FP16 128^3 43.5 / 52.2, 128x128x127 43.4 / 50.3, 256x128x64 42.0
+//   / 48.9; FP32 128x128x64 41.7 / 44.5, 192x128x128 140 / 149, 256x128x128 189 /
+//   200; 8 MiB alike: FP32 128^3 86.1 / 84.6).
+static bool deal4(const EsoParams& p, size_t word) {
+  const uint64_t n = p.n, box = (uint64_t)p.nx * p.ny * p.nz, row = n * word;
+  if (n + n / 64 < box) return true;
+  if (n < 65536) return false;
+  const uint64_t plane8 = n / p.nz + 128;  // (half a block up, so that near multiples count)
+  if (27 * row <= ((uint64_t)36 << 20) && plane8 % 2048 < 256 && plane8 % 8192 >= 256) return false;
+  const uint64_t mib4 = (uint64_t)4 << 20, near = row / 64, off = (row + near) % mib4;
+  return row < mib4 - near || row > 4 * mib4 + near || off > 2 * near;
+}
+
 template <class St>
 static int eso_update(psl_diad* d, bool child_records) {
   const EsoParams p = eso_params(d, child_records);
   const uint32_t nb = (uint32_t)((d->n + 255) / 256);
   typename St::T* f = (typename St::T*)d->f;
+  const bool four = deal4(p, sizeof(typename St::T));
+#define PSL_ESO_UPDATE(F, W)                                                  \
+  do {                                                                        \
+    if (four) k_eso_update<St, F, W, true><<<nb, 256, 0, d->stream>>>(f, p);  \
+    else k_eso_update<St, F, W, false><<<nb, 256, 0, d->stream>>>(f, p);      \
+  } while (0)
   if (wide_rows<typename St::T>(p.n)) {
-    if (d->flipper) k_eso_update<St, true, true><<<nb, 256, 0, d->stream>>>(f, p);
-    else k_eso_update<St, false, true><<<nb, 256, 0, d->stream>>>(f, p);
+    if (d->flipper) PSL_ESO_UPDATE(true, true);
+    else PSL_ESO_UPDATE(false, true);
   } else {
-    if (d->flipper) k_eso_update<St, true, false><<<nb, 256, 0, d->stream>>>(f, p);
-    else k_eso_update<St, false, false><<<nb, 256, 0, d->stream>>>(f, p);
+    if (d->flipper) PSL_ESO_UPDATE(true, false);
+    else PSL_ESO_UPDATE(false, false);
   }
+#undef PSL_ESO_UPDATE
   PSL_LAUNCH_CHECK();
   // the records this update wrote hold its values; the others are behind
   d->child.fresh = p.rec != nullptr;
