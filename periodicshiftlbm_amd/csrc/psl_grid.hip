@@ -597,6 +597,18 @@ static int listed_mode(const psl_grid* g) {
   return bytes < STAGE_FROM || bytes > to ? LIST_INLINE : LIST_STAGE;
 }
 
+// Between closure evaluations the listed cells are staged in every storage while
+// the grid is about as large as the last-level cache, and updated from their
+// slots beyond it, where the records add to the traffic (sphere channel, us per
+// held step, staged / slots, MB of the grid): FP32 26: 20.1 / 25.2, 184: 74.5 /
+// 80.4, 284: 134 / 143, 324: 171.3 / 171.9, 359: 194.0 / 191.5, 456: 253 / 242;
+// FP16 223: 95 / 101, 323: 190.3 / 190.5, 364: 216 / 208, 527: 328 / 314; BF16 223:
+// 96 / 102, 323: 191.3 / 192.8, 364: 216 / 210, 527: 329 / 316.
+constexpr size_t HELD_STAGE_TO = (size_t)336 << 20;
+static int held_listed_mode(const psl_grid* g) {
+  return 27ull * ncells(g) * storage_bytes(g->storage) > HELD_STAGE_TO ? LIST_NONE : LIST_STAGE;
+}
+
 static Faces faces_of(const psl_grid* g) {
   Faces f;
   f.x = (g->periodic_copies & 1) && g->info.cellCountX > 1 ? g->ring_x : nullptr;
@@ -662,8 +674,8 @@ static int launch_local_update(psl_grid* g, bool dominant_only = false, const Co
   }
   const int nt = g->tuning & (TUNE_NT_LOAD | TUNE_NT_STORE);
   const uint32_t nb = blocks_for(p.n);
-  // the network's own kernel updates them from their slots, held steps always stage them
-  const int list = !b.n || net || fused ? LIST_NONE : held ? LIST_STAGE : listed_mode(g);
+  // (the network's own kernel leaves them to k_ps_boundary)
+  const int list = !b.n || net || fused ? LIST_NONE : held ? held_listed_mode(g) : listed_mode(g);
   const bool copy = cstep.in || cstep.out;
   const Faces fc = faces_of(g);
   if (net) {
@@ -699,7 +711,7 @@ static int launch_local_update(psl_grid* g, bool dominant_only = false, const Co
     g->prof_events.emplace_back(ev0, ev1);
   }
   if (b.n && !fused && !dominant_only && list != LIST_INLINE) {
-    if (net) k_ps_boundary<St><<<blocks_for(b.n), 256, 0, g->stream>>>(p, b);
+    if (list != LIST_STAGE) k_ps_boundary<St><<<blocks_for(b.n), 256, 0, g->stream>>>(p, b);
     else {
       StagedParams sp;
       sp.f = g->f;

@@ -315,12 +315,15 @@ def test_held_closure_matches_oracle(psl, oracle_mod):
     assert e2_fresh > 10 * e2  # the held update did not evaluate the network
 
 
-@pytest.mark.parametrize("storage", ["f32", "f16", "bf16"])
-@pytest.mark.parametrize("shape,tuning", [((48, 24, 24), 4), ((37, 19, 23), 4), ((48, 24, 24), 3)])
+@pytest.mark.parametrize("storage,shape,tuning", [
+    *((st, shape, tuning) for st in ("f32", "f16", "bf16")
+      for shape, tuning in (((48, 24, 24), 4), ((37, 19, 23), 4), ((48, 24, 24), 3))),
+    ("f32", (162, 143, 145), 4)])
 def test_closure_steps_with_box_faces(psl, storage, shape, tuning):
     """A channel with inlet, outlet and solid cells under a constant network
     (y0 = 2, exact in FP16), evaluated every third step.  An evaluating step
-    (listed cells from their slots) and a held one (staged) from one state each
+    (listed cells from their slots) and a held one (staged, or from the slots on the
+    grid of 346 MB) from one state each
     leave the bits of the step without a closure in the listed and the solid
     cells (nu and Cs as set), and in the fluid ones the values at nu + 1e-3 y0
     without Smagorinsky: the viscosities' sums differ by a rounding, so within
