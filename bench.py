@@ -674,7 +674,8 @@ def main():
         out["variants"]["drag_history"] = dh
     if args.batch_steps:
         log(f"[bench] batch of 64 domains, {args.batch_steps} steps")
-        bl = batch_leg(P, cases, args.batch_steps, 0 if (args.no_autotune or args.tuning is not None) else 3)
+        # (20 steps per variant: calls of few steps run without groups)
+        bl = batch_leg(P, cases, args.batch_steps, 0 if (args.no_autotune or args.tuning is not None) else 20)
         log(f"  {bl['mlups']:.1f} MLUPS over {bl['cells']} cells")
         out["variants"]["batch"] = bl
     if args.large_n:

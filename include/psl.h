@@ -212,10 +212,10 @@ int psl_grid_get_tuning(const psl_grid* grid, int* tuning);
  * reference counterpart (a launch-shape setting, like the variants above). */
 int psl_grid_set_occupancy(psl_grid* grid, int workgroups_per_cu);
 int psl_grid_get_occupancy(const psl_grid* grid, int* workgroups_per_cu);
-/* Autotuner: times all PSL_TUNE_VARIANTS variants on this grid (`steps` whole
- * steps each after one warm-up: streaming, the grid's periodic copies and the
- * local update, so the rows are misaligned as in a run; the state and the
- * shifter advance); the variants within 2 % of the fastest are timed again
+/* Autotuner: times all PSL_TUNE_VARIANTS variants on this grid (one call of
+ * `steps` whole steps each after one warm-up: streaming, the grid's periodic
+ * copies and the local update, so the rows are misaligned as in a run and the
+ * copies go as in calls of that length; the state and the shifter advance); the variants within 2 % of the fastest are timed again
  * over max(steps, 256) steps (the time per step runs in phases tens of steps
  * long as the shifts carry the rows across lines and channels) and the
  * fastest of those is kept;
@@ -289,9 +289,10 @@ int psl_batch_get_steps_per_graph(const psl_batch* batch, int* steps);
 /* order 0: grids in the given order, 1: largest grid first (block order of the launch). */
 int psl_batch_set_tuning(psl_batch* batch, int tuning, int order);
 int psl_batch_get_tuning(const psl_batch* batch, int* tuning, int* order);
-/* Times the PSL_TUNE_VARIANTS variants x 2 orders (one warm-up step and `steps`
- * steps each; the grids advance) and keeps the fastest; times_ms[2 * PSL_TUNE_VARIANTS]
- * receives ms per step at order * PSL_TUNE_VARIANTS + variant. */
+/* Times the PSL_TUNE_VARIANTS variants x 2 orders (one warm-up step and one call of
+ * `steps` steps each; the grids advance) and keeps the fastest; times_ms[2 *
+ * PSL_TUNE_VARIANTS] receives ms per step at order * PSL_TUNE_VARIANTS + variant.
+ * Calls of few steps run without groups: tune with calls about as long as the run's. */
 int psl_batch_autotune(psl_batch* batch, int steps, int* best_tuning, int* best_order, double* times_ms);
 /* Layout of the two-launch bulk kernel: cells_per_thread 1 or 2 (a workgroup updates
  * 256 or 512 consecutive cells of one grid), tile_order 0 (each grid's tiles in turn)

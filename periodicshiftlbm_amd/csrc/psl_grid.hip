@@ -11,14 +11,17 @@
 //
 // Kernels of one step:
 //   k_ps_bulk      fluid + bounceback cells, one thread per cell, the hot path;
-//                  it also stages the box-face cells' loaded f (see Stage);
-//   k_ps_boundary_staged  box-face boundary cells from a compact list
-//                  (restore + MBBC + collision) on the staged f; the cell
-//                  sets are disjoint, so the two launches together equal the
-//                  reference's single update (k_ps_boundary: the same from
-//                  the slots, next to the learned-closure bulk kernel);
-//   k_ps_fused     both in one launch (a tuning variant);
-//   k_periodic     applyBCPeriodicX/Y surface copies (before the update).
+//                  it also updates the box-face boundary cells (restore + MBBC +
+//                  collision) in their own lanes, or stages their loaded f for a
+//                  second launch, by storage and size (listed_mode), and passes
+//                  the periodic copies of a multi-step call on (CopyStep);
+//   k_ps_boundary_staged  box-face cells from a compact list on the staged f;
+//                  the cell sets are disjoint, so the two launches together
+//                  equal the reference's single update (k_ps_boundary: the same
+//                  from the slots, next to the learned-closure bulk kernel);
+//   k_ps_fused     bulk and list workgroups in one launch (a tuning variant);
+//   k_periodic     applyBCPeriodicX/Y surface copies (before the update), where
+//                  they do not come through the ring.
 #include "psl_internal.h"
 #include "psl_stream.h"
 #include "psl_closure.h"
@@ -39,7 +42,8 @@ void set_error(const std::string& msg) { g_last_error = msg; }
 // lines 46-67: restore + MBBC + collision) and the bulk (fluid and
 // bounceback cells, in cell order).  After applyStreaming every cell owns its
 // 27 slots, so the two sets can be updated in any order or concurrently.
-//   k_ps_bulk + k_ps_boundary  two launches, one after the other;
+//   k_ps_bulk                  one launch, the listed cells in place, or two with
+//                              k_ps_boundary_staged / k_ps_boundary after it;
 //   k_ps_fused                 one launch in which each boundary-list
 //                              workgroup sits right before the bulk blocks
 //                              whose cells it covers (fused_order), so the
@@ -1446,10 +1450,6 @@ int psl_grid_get_tuning(const psl_grid* g, int* tuning) {
   return PSL_OK;
 }
 
-// Time every tuning variant of the bulk kernel on this grid (each for `steps`
-// updates with the grid's own data; the distributions advance by
-// 8 * steps updates) and keep the fastest.  times_ms (optional, 8 entries)
-// receives the mean bulk-kernel time of each variant.
 int psl_grid_set_occupancy(psl_grid* g, int workgroups_per_cu) {
   PSL_CHECK_ARG(g, "null grid");
   size_t lds = 0;
