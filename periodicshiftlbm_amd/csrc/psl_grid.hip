@@ -832,13 +832,20 @@ static int periodic_copy(psl_grid* g, int axis) {
 //   FP16 x in the cache, bound by VALU issue: 60 MB 30.4 / 29.2, 74 34.1 / 34.7,
 //   110 44.3 / 45.6, 156 57.4 / 57.8, 214 74.1 / 73.1 (BF16 x 35.2 / 34.8, 46.5 /
 //   45.8, 61.0 / 58.7; with y copies FP16 36.8 / 35.8, 46.8 / 46.8, 60.4 / 59.8);
-//   FP32 just beyond the cache: 219 MB 85.7 / 82.1, 263 131 / 135, 312 145 / 149,
-//   366 177 / 184, 427 208.0 / 209.1, 460 234 / 231, 530 281 / 269, 737 393 / 362.
+//   where the rings take the working set beyond the 256 MB last-level cache (how
+//   far below it depends on where the buffers lie), and in FP32 for a while after:
+//   FP32 219 MB 85.7 / 82.1, 230 89.9 / 89.4 to 113.8, 246 95.9 / 100.9, 252 98 /
+//   130, 263 131 / 135, 312 145 / 149, 366 177 / 184, 427 208.0 / 209.1, 460 234 /
+//   231, 530 281 / 269, 737 393 / 362;
+//   FP16 222 80.4 / 78.5, 238 84.5 / 82.1, 243 85 / 129, 256 90 / 144, 261 142 / 150,
+//   274 159 / 157, 304 170 / 166, 368 199 / 190;
+//   BF16 230 88.8 / 82.7, 238 92 / 120, 256 98 / 145, 265 152.8 / 151.5, 274 161 / 155.
 constexpr uint32_t RING_CELLS = 32768, RING_CELLS_16BIT = 70000;
 static bool ring_pays(const psl_grid* g) {
   const uint32_t n = ncells(g);
   const size_t mb = (27ull * n * storage_bytes(g->storage)) >> 20;
-  if (g->storage == PSL_F32) return n >= RING_CELLS && (mb < 240 || mb >= 448);
+  if (mb >= 224 && mb < (g->storage == PSL_F32 ? 448 : 272)) return false;
+  if (g->storage == PSL_F32) return n >= RING_CELLS;
   const bool y = (g->periodic_copies & 2) && g->info.cellCountY > 1;
   return n >= RING_CELLS_16BIT && (y || g->storage == PSL_BF16DEV || mb < 64 || mb >= 192);
 }
