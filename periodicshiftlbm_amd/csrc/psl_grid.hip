@@ -840,18 +840,24 @@ static int periodic_copy(psl_grid* g, int axis) {
 //   FP16 222 80.4 / 78.5, 238 84.5 / 82.1, 243 85 / 129, 256 90 / 144, 261 142 / 150,
 //   274 159 / 157, 304 170 / 166, 368 199 / 190;
 //   BF16 230 88.8 / 82.7, 238 92 / 120, 256 98 / 145, 265 152.8 / 151.5, 274 161 / 155.
+// The first step of a call pays for both, passes and ring, so inside the cache a
+// call has to be long enough (gain at 2 / 3 / 4 / 6 steps: FP32 147 MB 1.00 / 1.02 /
+// 1.03 / 1.04, x 0.98 / 1.00 / 1.01 / 1.01, 209 MB 0.96 / 0.98 / 0.99 / 1.00, x 0.95 /
+// 0.97 / 0.98 / 0.99; FP16 107 MB 0.98 / 0.99 / 0.99 / 1.00, x 5 MB 0.97 / 0.98 / 1.00
+// / 1.01; BF16 x 107 MB 0.97 / 0.98 / 0.99 / 1.00; elsewhere 2 steps gain 0 to 11 %).
 constexpr uint32_t RING_CELLS = 32768, RING_CELLS_16BIT = 70000;
-static bool ring_pays(const psl_grid* g) {
+static bool ring_pays(const psl_grid* g, int steps) {
   const uint32_t n = ncells(g);
   const size_t mb = (27ull * n * storage_bytes(g->storage)) >> 20;
   if (mb >= 224 && mb < (g->storage == PSL_F32 ? 448 : 272)) return false;
-  if (g->storage == PSL_F32) return n >= RING_CELLS;
   const bool y = (g->periodic_copies & 2) && g->info.cellCountY > 1;
+  if (g->storage == PSL_F32) return n >= RING_CELLS && (mb < 128 || mb >= 224 || steps >= (y ? 6 : 16));
+  if (mb < 224 && (mb >= 64 || !y) && steps < 4) return false;
   return n >= RING_CELLS_16BIT && (y || g->storage == PSL_BF16DEV || mb < 64 || mb >= 192);
 }
-static bool ring_runs(const psl_grid* g) {
-  return (g->periodic_copies & 1) && g->info.cellCountX > 1 && !g->census[2] && !g->closure &&
-         !(g->flags && g->n_bc) && ring_pays(g);
+static bool ring_runs(const psl_grid* g, int steps) {
+  return steps > 1 && (g->periodic_copies & 1) && g->info.cellCountX > 1 && !g->census[2] && !g->closure &&
+         !(g->flags && g->n_bc) && ring_pays(g, steps);
 }
 
 // The rings of the grid's copied faces, made when a call first uses them;
@@ -880,7 +886,7 @@ static bool ensure_rings(psl_grid* g) {
          make(&g->ring_x, 4 * (size_t)I.cellCountY * I.cellCountZ * X_RUN * esz);
 }
 int grid_steps(psl_grid* g, int steps) {
-  const bool ring = steps > 1 && ring_runs(g) && ensure_rings(g);
+  const bool ring = ring_runs(g, steps) && ensure_rings(g);
   CopyStep c{0u, false, false};
   for (int s = 0; s < steps; ++s) {
     int rc = psl_apply_streaming(g);
