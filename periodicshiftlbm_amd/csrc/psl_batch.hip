@@ -270,15 +270,21 @@ bool fused_form(const psl_batch* b) { return (b->tuning & PSL_TUNE_FUSED_BOUNDAR
 //   4 / 20; 274 MB 1.06 at 20, 321 MB 1.03, 374 MB 0.99, 432 MB 0.96;
 //   FP16 with lists gains at every length and size, the lists find their grid's
 //   lines again: 60 channels 1.13 / 1.35 at 2 / 20; 271 MB 1.06, 562 MB 1.04.
+// A batch of up to `whole` bytes still stays in the cache in one piece (gain at 60
+// steps, batches of 4 to 19 grids: FP16 with lists 194 MB 0.99, 203 0.95, 216 0.98,
+// 222 0.97, 228 1.22; 16 bits fused 194 1.00 to 1.11, 203 0.98 to 1.04, 209 1.01 to
+// 1.08, 222 1.19; BF16 in place 194 1.01, 209 0.98, 216 1.03; FP32 in place 192
+// 1.03, fused 192 0.99, 203 0.99 to 1.02, 215 1.04).
 struct GroupRule {
   int steps;
-  size_t lone;
+  size_t lone, whole;
 };
 GroupRule group_rule(const psl_batch* b) {
   const size_t mb = (size_t)1 << 20;
-  if (b->storage == PSL_F32) return {4, 348 * mb};
-  if (fused_form(b)) return {6, 248 * mb};
-  return lists_in_place(b) || !b->total_bnd ? GroupRule{4, 248 * mb} : GroupRule{2, SIZE_MAX};
+  const bool fused = fused_form(b);
+  if (b->storage == PSL_F32) return {4, 348 * mb, (fused ? 208 : 192) * mb};
+  if (fused) return {6, 248 * mb, 208 * mb};
+  return lists_in_place(b) || !b->total_bnd ? GroupRule{4, 248 * mb, 212 * mb} : GroupRule{2, SIZE_MAX, 224 * mb};
 }
 
 // Step s of a run of `steps` steps of one group of grids.
@@ -445,7 +451,11 @@ int build_batch(psl_batch* b) {
   b->launch_order.assign(order.begin(), order.end());
   std::vector<size_t> bytes;
   for (int d : order) bytes.push_back((size_t)b->grids[d]->info.cellCount * 27 * storage_bytes(b->storage));
-  const std::vector<size_t> ends = group_ends(bytes, GROUP_BYTES, group_rule(b).lone);
+  const GroupRule rule = group_rule(b);
+  size_t total = 0;
+  for (size_t x : bytes) total += x;
+  const std::vector<size_t> ends =
+      total <= rule.whole ? std::vector<size_t>{bytes.size()} : group_ends(bytes, GROUP_BYTES, rule.lone);
   std::vector<BatchEntry> fused;
   size_t at0 = 0;
   b->groups.clear();
