@@ -266,9 +266,9 @@ int psl_grid_check_health(psl_grid* grid, int64_t* bad_cells, double* rho_min, d
  * (FP16) one launch over all boundary lists, or one fused launch.  Steps are
  * captured in hipGraphs of one step and of steps_per_graph steps (default 1000)
  * and replayed, so nsteps steps take nsteps / steps_per_graph + nsteps %
- * steps_per_graph graph launches; a batch whose distributions exceed 192 to 224 MB
- * instead takes calls of several steps (from 2, 4 or 6 on; both by storage and
- * variant) in groups of grids that fit the last-level cache, all steps of one
+ * steps_per_graph graph launches; a batch whose distributions exceed 192 MB (FP16
+ * with two launches 224 MB) instead takes calls of several steps (from 2, 4 or 6
+ * on, by storage and variant) in groups of grids that fit the last-level cache, all steps of one
  * group after the other, launched without a graph.  Every grid's result is
  * bit-identical to stepping it alone.  After a launch error every grid's
  * shifter stands at the steps launched for it.  Grids need flags and

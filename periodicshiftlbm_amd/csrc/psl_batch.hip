@@ -270,21 +270,22 @@ bool fused_form(const psl_batch* b) { return (b->tuning & PSL_TUNE_FUSED_BOUNDAR
 //   4 / 20; 274 MB 1.06 at 20, 321 MB 1.03, 374 MB 0.99, 432 MB 0.96;
 //   FP16 with lists gains at every length and size, the lists find their grid's
 //   lines again: 60 channels 1.13 / 1.35 at 2 / 20; 271 MB 1.06, 562 MB 1.04.
-// A batch of up to `whole` bytes still stays in the cache in one piece (gain at 60
-// steps, batches of 4 to 19 grids: FP16 with lists 194 MB 0.99, 203 0.95, 216 0.98,
-// 222 0.97, 228 1.22; 16 bits fused 194 1.00 to 1.11, 203 0.98 to 1.04, 209 1.01 to
-// 1.08, 222 1.19; BF16 in place 194 1.01, 209 0.98, 216 1.03; FP32 in place 192
-// 1.03, fused 192 0.99, 203 0.99 to 1.02, 215 1.04).
+// A batch of up to `whole` bytes is stepped in one piece: with FP16's lists it
+// still stays in the cache (gain of groups at 60 steps, batches of 4 to 19 grids:
+// 194 MB 0.99, 203 0.95, 216 0.98, 222 0.97, 228 1.22); in the other forms that
+// depends on where the buffers lie, and groups lose at most 2 % from 192 MB on
+// (16 bits fused 194 MB 1.00 to 1.11, 203 0.98 to 1.04, 222 1.19; BF16 in place 194
+// 1.01, 205 1.01 to 1.08, 209 0.98, 216 1.03; FP32 in place 192 1.03, fused 192
+// 0.99, 203 0.99 to 1.02, 215 1.04).
 struct GroupRule {
   int steps;
   size_t lone, whole;
 };
 GroupRule group_rule(const psl_batch* b) {
   const size_t mb = (size_t)1 << 20;
-  const bool fused = fused_form(b);
-  if (b->storage == PSL_F32) return {4, 348 * mb, (fused ? 208 : 192) * mb};
-  if (fused) return {6, 248 * mb, 208 * mb};
-  return lists_in_place(b) || !b->total_bnd ? GroupRule{4, 248 * mb, 212 * mb} : GroupRule{2, SIZE_MAX, 224 * mb};
+  if (b->storage == PSL_F32) return {4, 348 * mb, GROUP_BYTES};
+  if (fused_form(b)) return {6, 248 * mb, GROUP_BYTES};
+  return lists_in_place(b) || !b->total_bnd ? GroupRule{4, 248 * mb, GROUP_BYTES} : GroupRule{2, SIZE_MAX, 224 * mb};
 }
 
 // Step s of a run of `steps` steps of one group of grids.
