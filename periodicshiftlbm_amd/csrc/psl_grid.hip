@@ -827,8 +827,9 @@ static int periodic_copy(psl_grid* g, int axis) {
 // The sizes (us per step of a cubic box, passes / ring; x: no y copies):
 //   a small step is bound by latency, most of it fetching the kernels'
 //   instructions: FP32 33x33x32 12.9 / 12.4, 41x41x40 14.0 / 12.9, FP16 17x17x16
-//   12.4 / 13.7, 33x33x32 12.9 / 13.1, 41x41x40 13.6 / 13.5, 49x49x48 14.7 / 13.7, x
-//   37x36x36 10.6 / 11.1, 41x40x40 11.3 / 11.4, 45x44x44 11.8 / 11.6;
+//   12.4 / 13.7, 33x33x32 12.9 / 13.1, 37x37x36 14.2 / 12.4, 41x41x40 13.6 / 13.5 to
+//   14.9 / 12.9, 49x49x48 14.7 / 13.7, x 37x36x36 10.6 / 11.1, 41x40x40 11.3 / 11.4,
+//   45x44x44 11.8 / 11.6;
 //   FP16 x in the cache, bound by VALU issue: 60 MB 30.4 / 29.2, 74 34.1 / 34.7,
 //   110 44.3 / 45.6, 156 57.4 / 57.8, 214 74.1 / 73.1 (BF16 x 35.2 / 34.8, 46.5 /
 //   45.8, 61.0 / 58.7; with y copies FP16 36.8 / 35.8, 46.8 / 46.8, 60.4 / 59.8);
@@ -845,7 +846,7 @@ static int periodic_copy(psl_grid* g, int axis) {
 // 1.03 / 1.04, x 0.98 / 1.00 / 1.01 / 1.01, 209 MB 0.96 / 0.98 / 0.99 / 1.00, x 0.95 /
 // 0.97 / 0.98 / 0.99; FP16 107 MB 0.98 / 0.99 / 0.99 / 1.00, x 5 MB 0.97 / 0.98 / 1.00
 // / 1.01; BF16 x 107 MB 0.97 / 0.98 / 0.99 / 1.00; elsewhere 2 steps gain 0 to 11 %).
-constexpr uint32_t RING_CELLS = 32768, RING_CELLS_16BIT = 70000;
+constexpr uint32_t RING_CELLS = 32768, RING_CELLS_16BIT = 45000, RING_CELLS_16BIT_X = 70000;
 static bool ring_pays(const psl_grid* g, int steps) {
   const uint32_t n = ncells(g);
   const size_t mb = (27ull * n * storage_bytes(g->storage)) >> 20;
@@ -853,7 +854,8 @@ static bool ring_pays(const psl_grid* g, int steps) {
   const bool y = (g->periodic_copies & 2) && g->info.cellCountY > 1;
   if (g->storage == PSL_F32) return n >= RING_CELLS && (mb < 128 || mb >= 224 || steps >= (y ? 6 : 16));
   if (mb < 224 && (mb >= 64 || !y) && steps < 4) return false;
-  return n >= RING_CELLS_16BIT && (y || g->storage == PSL_BF16DEV || mb < 64 || mb >= 192);
+  return n >= (y ? RING_CELLS_16BIT : RING_CELLS_16BIT_X) &&
+         (y || g->storage == PSL_BF16DEV || mb < 64 || mb >= 192);
 }
 static bool ring_runs(const psl_grid* g, int steps) {
   return steps > 1 && (g->periodic_copies & 1) && g->info.cellCountX > 1 && !g->census[2] && !g->closure &&

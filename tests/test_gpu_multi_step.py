@@ -33,7 +33,7 @@ def _same(a, b, what):
     assert nbad == 0, f"{what}: {nbad} values differ"
 
 
-# (from 32768 cells on, FP32; 16-bit grids from 70000 on) rows shorter than, equal to and longer than a wave and a
+# (from 32768 cells on, FP32; 16-bit grids from 45000 or 70000 on) rows shorter than, equal to and longer than a wave and a
 # workgroup; single and double layers on every axis, where a copied face is its
 # own or its neighbour's
 SHAPES = [(2, 130, 128), (3, 200, 60), (5, 100, 70), (17, 50, 41), (63, 3, 180), (64, 4, 130), (65, 5, 110),
